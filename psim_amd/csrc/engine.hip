@@ -4,13 +4,14 @@
 // Data layout in HBM:
 //   model      cells, edges (3 per cell), sub-surfaces, sensors, materials, frequency/velocity
 //              arrays and the CDF / LA-fraction tables: uploaded once, read-only, L2-resident.
-//   pool       emission output, one slot per phonon id, structure of arrays: px py dx dy freq vel
-//              age tts (f64), cell (i32, -1 = never starts), meta (u32: bin, polarization, sign,
-//              started, rate sensor).  Read once, when the phonon's birth window fetches it.
+//   pool       emission output, one slot per phonon id: a 64-byte record (position, direction,
+//              frequency, velocity, birth time, cell, sensor) and two words (meta: bin,
+//              polarization, sign, stream; id in its stream).  Read once, when the phonon's birth
+//              window fetches it.
 //   tallies    counts [S][R] (i64) and flux [S][R][2] (f64), as Sensor::inc_energy_/inc_flux_.
 //   partials   per transport block: [W][S] count (i32) and flux (2 x f64) of one launch window.
 //
-//   live       two dense buffers with the pool's fields plus the phonon id: each transport launch
+//   live       two dense buffers of 96-byte records with the phonon's whole state: each transport launch
 //              reads the survivors of the previous window from one, in order, plus the phonons
 //              born in its own window (ids sorted by birth step, counting sort), and appends its
 //              survivors to the other.
@@ -176,10 +177,8 @@ __global__ void __launch_bounds__(BLOCK) emit_kernel(Model m, Pool pool, int64_t
             key = (int32_t)step;
         }
         birth_key[id] = key;
-        pool.pos[id] = make_double2(p.px, p.py);
-        pool.dir[id] = make_double2(p.dx, p.dy);
-        pool.fv[id] = make_double2(p.freq, p.vel);
-        pool.aux[id] = PoolAux{ birth, cell, cl.sensor };
+        pool.rec[id] = PoolRec{ make_double2(p.px, p.py), make_double2(p.dx, p.dy), make_double2(p.freq, p.vel), birth,
+            cell, cl.sensor };
         pool.ms[id] = make_uint2((uint32_t)p.bin | (p.pol == POL_TA ? META_TA : 0u) | (p.sign < 0 ? META_NEG : 0u)
                                      | ((uint32_t)src.stream << META_STREAM_SHIFT),
             sid);
@@ -245,30 +244,23 @@ __global__ void __launch_bounds__(BLOCK) birth_scatter_kernel(const int32_t* __r
 // State of the phonons that are alive between two launch windows, densely packed in the order
 // the previous launch paused them, with the phonon id (the key of its Philox stream).  A launch
 // reads its started phonons from one buffer in work-queue order and appends its survivors to the
-// other, so the phonons that neighbouring lanes and waves fetch or park share cache lines.  Seven
-// arrays of 16-byte records (112 B per phonon): a lane moves a phonon in seven vector loads or
-// stores, and a launch holds seven pointers per buffer.
-struct __attribute__((aligned(16))) LiveAux {
-    double rate2;  // third relaxation rate of the last scattering-time draw
-    int32_t cell;  // -1: a hole (a reserved slot nobody filled)
+// other.  One 96-byte record per phonon: a wave seldom refills more than a few lanes at once
+// (1.3-5 measured), so a record of its own cache lines beats arrays of fields, whose lines the lane
+// shares with phonons that other waves fetch later.  The cell stands apart, for the sort.
+struct __attribute__((aligned(16))) LiveRec {
+    double2 pos, dir;
+    double2 fv;  // freq, vel
+    double2 at;  // age, time to the next scatter
+    double2 ab;  // the shares Rates::a, Rates::b of the last scattering-time draw
+    uint32_t meta;
+    uint32_t id;
+    int32_t step;  // measurement step (past the window's end after a long flight)
     int32_t sensor;  // sensor of the cell
 };
 
-struct __attribute__((aligned(16))) LiveTag {
-    uint32_t meta;
-    uint32_t id;
-    uint32_t sid;  // id within the phonon's random stream
-    int32_t step;  // measurement step (past the window's end after a long flight)
-};
-
 struct Live {
-    double2* __restrict__ pos;  // px, py
-    double2* __restrict__ dir;  // dx, dy
-    double2* __restrict__ fv;  // freq, vel
-    double2* __restrict__ at;  // age, time to the next scatter
-    double2* __restrict__ r01;  // first two relaxation rates of the last scattering-time draw
-    LiveAux* __restrict__ aux;
-    LiveTag* __restrict__ tag;
+    LiveRec* __restrict__ rec;
+    uint2* __restrict__ cell;  // cell (-1: a hole, a reserved slot nobody filled), id in the phonon's stream
 };
 
 // Work of one transport launch: the started phonons (Live buffer `in`, *n_in entries) followed by
@@ -302,17 +294,28 @@ constexpr int TALLY_NONE = 0, TALLY_LDS = 1, TALLY_GLOBAL = 2;
 #define PSIM_TRANSPORT_WAVES_PER_EU 2
 #endif
 
+// Events of one wave, wave-uniform: counted from the stage masks in scalar registers.
+struct WaveCounters {
+    uint64_t scatters, impacts;
+    uint32_t relocations, absorbed, expired, stalled;
+};
+
 // Lane states of the scheduled event loop.
-enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_END = 5, S_EXIT = 6, S_PAUSED = 7, S_DEAD = 8 };
+enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_WALL = 5, S_END = 6, S_EXIT = 7, S_PAUSED = 8,
+    S_DEAD = 9 };
 
 // Advances the listed phonons across measurement steps [k0, k1).  Each lane carries one phonon
 // through ModelSimulator::simulatePhonon (psim/src/modelSimulator.cpp:139-198), pausing right
 // after the measurement that brings its step to k1, then takes the next phonon of the launch's
-// work queue.  The loop is split into stages -- fetch, surface handling after a hit, scatter and
-// the scattering-time draw, one nextImpact -- and every iteration of the wave runs them in that
-// order, each for the lanes waiting in it, so lanes that finish one stage join the next in the
-// same iteration.  Each lane still performs exactly the reference's sequence of operations for
-// its phonon, so trajectories are unchanged.
+// work queue.  The loop is split into stages -- fetch, one nextImpact, the surface a hit lies on,
+// the end of a drift, the draws (scatters, scattering times, reflections) -- and every iteration of
+// the wave runs them in that order, each for the lanes waiting in it, so lanes that finish one
+// stage join the next in the same iteration.  Each lane still performs exactly the reference's
+// sequence of operations for its phonon, so trajectories are unchanged.
+// Bound: VALU issue (80% of the cycles in the untallied variant, 35 of 64 lanes active).  1e7
+// phonons of the L-shape: 1122 vector instructions per wave iteration, untallied launch 149.7 ms of
+// kernels in all, the run 158.7 ms; with reflections done inside the surface search, divisors not
+// shared, coefficients and buffer pointers spilled to vector lanes: 1580 and 200.2 ms.
 // TALLY: the tally path of this launch (TALLY_NONE, TALLY_LDS, TALLY_GLOBAL).
 // MULTI: some source has a stream index or id base (a batch of models).  Otherwise a phonon's
 // id within its stream is its id and the stream word is the bare tag, so the single-model
@@ -320,12 +323,37 @@ enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_END = 5
 // both variants draw the same numbers for such a model.
 // NT: threads per block (128, 256 or 512), a launch shape the autotuner chooses.
 // FT: the flux tallies' element type, double or float (FP32 with Kahan-compensated sums).
+// The kernel's one argument.  What the event loop reads all the time is taken from it once; the
+// rest (buffers that only refills, pauses and ends touch) is read again from the argument segment
+// where it is used (cold()): kept in scalar registers all along, those pointers crowded out the
+// loop's own values, which then went to and from the lanes of a vector register in every stage.
+struct Args {
+    Model m;
+    Pool pool;
+    Lists lists;
+    Tally tally;
+    Fate fate;
+    const uint64_t* __restrict__ seed_p;
+    unsigned long long* __restrict__ counters;
+    int32_t k0, k1;
+};
+
+typedef const __attribute__((address_space(4))) Args* ArgsPtr;
+
+__device__ __forceinline__ ArgsPtr cold() {
+    ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));  // opaque: loads through it stay where they are written
+    return p;
+}
+
 template <int TALLY, bool MULTI, int NT, typename FT>
 __global__ void __launch_bounds__(NT)
 __attribute__((amdgpu_waves_per_eu(TALLY == TALLY_NONE ? PSIM_UNTALLIED_WAVES_PER_EU : PSIM_TRANSPORT_WAVES_PER_EU)))
-transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const uint64_t* __restrict__ seed_p,
-    Tally tally, unsigned long long* __restrict__ counters, Fate fate) {
-    const uint64_t seed = *seed_p;
+transport_kernel(Args args) {
+    const Model& m = args.m;
+    const Tally& tally = args.tally;
+    const int32_t k0 = args.k0, k1 = args.k1;
+    const uint64_t seed = *args.seed_p;
     extern __shared__ unsigned char lds_raw[];
     const int S = m.n_sensors;
     // LDS window tallies as difference arrays over the window's steps: a flight that passes
@@ -343,13 +371,13 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     }
     __syncthreads();
 
-    LaneCounters c = { 0, 0, 0, 0, 0, 0, 0, 0 };
+    WaveCounters wc = { 0, 0, 0, 0, 0, 0 };
+    uint32_t n_steps = 0, n_tallies = 0;  // this lane's phonon-steps and tallies
     const int lane = threadIdx.x % WAVE;
     const uint64_t lane_below = (1ull << lane) - 1ull;
-    const int64_t n_live = *lists.n_in;
-    const int64_t b0 = lists.born_offset[k0];
-    const int64_t n_items = n_live + (int64_t)lists.born_offset[k1] - b0;
-    uint32_t* __restrict__ queue = lists.queue + lists.window;
+    const int64_t n_live = *args.lists.n_in;
+    const int64_t b0 = args.lists.born_offset[k0];
+    const int64_t n_items = n_live + (int64_t)args.lists.born_offset[k1] - b0;
 
     int state = S_FETCH;
     uint32_t slot = 0;
@@ -358,18 +386,27 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     p.cell = p.bin = p.pol = 0;
     p.sign = 1;
     p.step = 0;
-    double age = 0., tts = 0., ttm = 0.;
-    double relax[3] = { 0., 0., 0. };
+    double age = 0., tts = 0.;
+    Rates rates = { 0., 0., false };
     int events = 0;
     double drift_time = 0., drifted = 0., t_hit = 0.;
     int sensor0 = 0, collisions = 0;
     int cur_sensor = 0;  // sensor of p.cell
-    psim_stream st;
-    psim_stream_init(&st, seed, PSIM_TAG_TRANSPORT, 0, 0);
+    int wall = 0;  // S_WALL: the surface to reflect off (surface_hit)
+    bool passed = false;  // S_WALL: nothing to reflect off, only to be relocated
+    // The phonon's random stream: its next block, its id in the stream and (batches) its counter
+    // word; the step word is p.step.
+    uint32_t block = 0, sid = 0, tag = PSIM_TAG_TRANSPORT;
+    auto stream = [&]() -> psim_stream {
+        return psim_stream{ (uint32_t)seed, (uint32_t)(seed >> 32), (uint32_t)p.step, sid,
+            MULTI ? tag : PSIM_TAG_TRANSPORT, block };
+    };
     // Only untallied launches hold phonons below `stop`: every window that records starts at step
     // adj - 1 = stop or later.
     const int32_t stop = TALLY == TALLY_NONE ? m.stop : 0;
     const double steps_per_time = (double)m.N / m.sim_time;
+    const double dN = (double)m.N;
+    auto boundary_time = [&](int32_t k) -> double { return div_by((double)k * m.sim_time, dN, m.r_N); };  // k * sim_time / N
     // A flight ends at boundary `stop` (steady state, while the step lies below it), from there on at
     // every cap_len-th boundary after it (the model's flight cap), and at boundary N.  `cap` is the
     // current flight's cap, set when a phonon is fetched and when a flight reaches its cap.
@@ -388,7 +425,7 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     // stall bound, S_TTS when a scattering time is due (drawn once, then drift_setup), else
     // drift_setup directly.
     auto drift_setup = [&]() {
-        ttm = (double)cap * m.sim_time / (double)m.N - age;  // time to the flight's cap
+        const double ttm = boundary_time(cap) - age;  // time to the flight's cap
         drift_time = (ttm < tts) ? ttm : tts;
         sensor0 = cur_sensor;
         drifted = 0.;
@@ -397,7 +434,6 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     };
     auto begin_event = [&]() {
         if (++events > PSIM_MAX_EVENTS_PER_STEP) {
-            c.stalled++;
             state = S_DEAD + FATE_STALLED * 8;
             return;
         }
@@ -432,6 +468,7 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
                 }
             }
             if (first <= last) {
+                const Tally& tally = args.tally;
                 const int64_t row = (int64_t)cur_sensor * (m.R + 1) - m.adj;
                 const int64_t t0 = row + first, t1 = row + last + 1;
                 atomicAdd(reinterpret_cast<unsigned long long*>(&tally.dcnt[t0]), (unsigned long long)(int64_t)p.sign);
@@ -443,7 +480,7 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
                 atomicAdd(&dfy[t0], (FT)vy);
                 atomicAdd(&dfy[t1], (FT)-vy);
             }
-            c.tallies += (uint32_t)(last - a + 1);
+            n_tallies += (uint32_t)(last - a + 1);
         }
     };
     // The measurement events of the boundaries a flight passed up to time t
@@ -455,13 +492,13 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
         int32_t k = p.step;
         const int32_t est = (int32_t)(t * steps_per_time) - 1;  // a whole step below t: at or below the answer
         if (est > k) { k = est < cap - 1 ? est : cap - 1; }
-        while (k + 1 < cap && (double)(k + 1) * m.sim_time / (double)m.N <= t) { ++k; }
+        while (k + 1 < cap && boundary_time(k + 1) <= t) { ++k; }
         if (k == p.step) { return false; }
         if constexpr (TALLY != TALLY_NONE) { tally_range(p.step + 1 > m.adj ? p.step + 1 : m.adj, k); }
-        c.steps += (uint32_t)(k - p.step);
+        n_steps += (uint32_t)(k - p.step);
         p.step = k;
         events = 0;
-        psim_stream_set_step(&st, (uint32_t)k);
+        block = 0;
         return true;
     };
     // The rest of simulatePhonon's loop body once handleImpacts returned `result`, with the
@@ -470,36 +507,35 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     // with no draw made (so a resumed phonon continues exactly), at the latest at boundary
     // `stop`, where every window before the recorded steps ends.
     bool relocated = false;  // the flight ended frozen after a relocation (same sensor, same scattering time)
-    double end_arg = 0.;  // S_END: handleImpacts' result, applied by end_drift
-    auto end_drift = [&](double result) {
-        if (cur_sensor != sensor0) { drift_time = result; }
-        const double factor = p.vel * (drift_time - result);  // Phonon::drift
+    // `drifted` is handleImpacts' result here.
+    auto end_drift = [&]() {
+        const double ttm = boundary_time(cap) - age;  // as drift_setup had it: neither moved since
+        if (cur_sensor != sensor0) { drift_time = drifted; }
+        const double factor = p.vel * (drift_time - drifted);  // Phonon::drift
         p.px += p.dx * factor;
         p.py += p.dy * factor;
         age += drift_time;
-        ttm -= drift_time;
+        const double left = ttm - drift_time;
         tts -= drift_time;
         const bool advanced = advance_step(age, cap);
-        if (ttm == 0. && cap == m.N) {  // boundary N: the run is over (step_times_ has N entries)
-            c.steps++;
-            c.expired++;
-            p.step = m.N;
-            state = S_DEAD + FATE_EXPIRED * 8;
-            return;
-        }
-        if (ttm == 0.) {  // the flight reached boundary `cap`
-            c.steps++;
+        if (left == 0.) {  // the flight reached boundary `cap`
+            n_steps++;
+            if (cap == m.N) {  // boundary N: the run is over (step_times_ has N entries)
+                p.step = m.N;
+                state = S_DEAD + FATE_EXPIRED * 8;
+                return;
+            }
             if constexpr (TALLY != TALLY_NONE) {
                 if (cap >= m.adj) { tally_range(cap, cap); }
             }
             p.step = cap;
             events = 0;
-            psim_stream_set_step(&st, (uint32_t)cap);
-            cap = cap_for(p.step);
+            block = 0;
             if (p.step >= k1) {
                 state = S_PAUSED;
                 return;
             }
+            cap = cap_for(p.step);
         } else {
             if (!m.phasor && tts == 0.) {
                 state = S_SCAT;
@@ -529,7 +565,7 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
             const uint32_t take = need > QUEUE_CLAIM ? need : QUEUE_CLAIM;
             const int leader = __ffsll((unsigned long long)m_fetch) - 1;
             uint32_t base = 0;
-            if (lane == leader) { base = atomicAdd(queue, take); }
+            if (lane == leader) { base = atomicAdd(cold()->lists.queue + cold()->lists.window, take); }
             base = __shfl(base, leader, WAVE);
             item = rank < avail ? (int64_t)res_next + rank : (int64_t)base + (rank - avail);
             res_next = base + need;
@@ -540,42 +576,38 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
                 state = S_EXIT;
             } else {
                 // started phonons from the dense buffer, phonons born in the window from the pool
-                const bool started = item < n_live;
-                const Live& L = lists.in;
-                uint32_t meta, sid;
+                uint32_t meta;
                 double2 pos, dir, fv;
-                if (started) {
-                    const LiveTag tg = L.tag[item];
-                    slot = tg.id;
-                    meta = tg.meta;
-                    sid = tg.sid;
-                    p.step = tg.step;
-                    pos = L.pos[item];
-                    dir = L.dir[item];
-                    fv = L.fv[item];
-                    const double2 at = L.at[item];
+                if (item < n_live) {
+                    const LiveRec& L = cold()->lists.in.rec[item];
+                    const uint2 cs = cold()->lists.in.cell[item];
+                    slot = L.id;
+                    meta = L.meta;
+                    p.step = L.step;
+                    pos = L.pos;
+                    dir = L.dir;
+                    fv = L.fv;
+                    const double2 at = L.at, ab = L.ab;
                     age = at.x;
                     tts = at.y;
-                    const double2 r = L.r01[item];  // rates of the last scattering-time draw
-                    const LiveAux ax = L.aux[item];
-                    relax[0] = r.x;
-                    relax[1] = r.y;
-                    relax[2] = ax.rate2;
-                    p.cell = ax.cell;
-                    cur_sensor = ax.sensor;
+                    rates.a = ab.x;
+                    rates.b = ab.y;
+                    p.cell = (int32_t)cs.x;
+                    sid = cs.y;
+                    cur_sensor = L.sensor;
                 } else {  // a new phonon has no scattering time and no rates yet
-                    slot = lists.born_order[b0 + (item - n_live)];
-                    const uint2 ms = pool.ms[slot];
+                    slot = cold()->lists.born_order[b0 + (item - n_live)];
+                    const uint2 ms = cold()->pool.ms[slot];
+                    const PoolRec& L = cold()->pool.rec[slot];
                     meta = ms.x;
                     sid = ms.y;
-                    pos = pool.pos[slot];
-                    dir = pool.dir[slot];
-                    fv = pool.fv[slot];
-                    const PoolAux ax = pool.aux[slot];
-                    age = ax.age;
+                    pos = L.pos;
+                    dir = L.dir;
+                    fv = L.fv;
+                    age = L.age;
                     tts = 0.;
-                    p.cell = ax.cell;
-                    cur_sensor = ax.sensor;
+                    p.cell = L.cell;
+                    cur_sensor = L.sensor;
                     p.step = (int32_t)(age / m.step_time);
                 }
                 if (!MULTI) { sid = slot; }
@@ -587,15 +619,12 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
                 p.dy = dir.y;
                 p.freq = fv.x;
                 p.vel = fv.y;
-                p.bin = (int)(meta & META_BIN_MASK);
                 p.pol = (meta & META_TA) ? POL_TA : POL_LA;
                 p.sign = (meta & META_NEG) ? -1 : 1;
-                ttm = 0.;
+                rates.impurity = (meta & META_IMPURITY) != 0;
                 events = 0;
-                // the stream keeps (stream index, id within it) in its counter words c3 and c2
-                psim_stream_init(&st, seed,
-                    MULTI ? psim_stream_tag(PSIM_TAG_TRANSPORT, meta >> META_STREAM_SHIFT) : PSIM_TAG_TRANSPORT, sid,
-                    (uint32_t)p.step);
+                block = 0;
+                if (MULTI) { tag = psim_stream_tag(PSIM_TAG_TRANSPORT, meta >> META_STREAM_SHIFT); }
                 if (p.step >= k1) {  // a long flight already carried it past this window
                     state = S_PAUSED;
                 } else {
@@ -607,52 +636,24 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     // One nextImpact of handleImpacts.
     auto stage_ni = [&]() {
         if (state == S_NI) {  // one nextImpact of handleImpacts
-            if (find_impact(m, p, drift_time - drifted, t_hit, c)) {
-                state = S_COLL;
-            } else {
-                end_arg = drifted;
-                state = S_END;
-            }
+            state = find_impact(m, p, drift_time - drifted, t_hit) ? S_COLL : S_END;
         }
     };
-    // Surface handling after a hit, then handleImpacts' bookkeeping.
+    // The surface a hit lies on, and handleImpacts' bookkeeping.  A phonon that reflects goes on to
+    // the draws stage (S_WALL), as does one due for relocation.
     auto stage_coll = [&]() {
-        if (state == S_COLL) {  // surface handling, then handleImpacts' bookkeeping
+        if (state == S_COLL) {
             // the boundaries passed before the impact see the old direction; the surface sees
             // the step of the moment of impact
             // the reference counts collisions per drift, and a drift ends at a boundary
             if (advance_step(age + (drifted + t_hit), cap)) { collisions = 0; }
-            handle_surface_collision(m, p, p.px, p.py, st);
-            if (p.cell < 0) {
-                c.absorbed++;
+            const int hit = surface_hit(m, p, cur_sensor, wall);
+            if (hit == HIT_ABSORBED) {
                 state = S_DEAD + FATE_ABSORBED * 8;
             } else {
-                cur_sensor = m.cells[p.cell].sensor;
                 drifted += t_hit;
-                if (++collisions > MAX_COLLISIONS) {  // Phonon::setRandPoint -> Triangle::getRandPoint
-                    double r1, r2;
-                    psim_urand2(&st, &r1, &r2);
-                    const psim_cell& cl = m.cells[p.cell];
-                    if (r1 + r2 > 1.) {
-                        r1 = 1 - r1;
-                        r2 = 1 - r2;
-                    }
-                    p.px = cl.x1 + (cl.x2 - cl.x1) * r1 + (cl.x3 - cl.x1) * r2;
-                    p.py = cl.y1 + (cl.y2 - cl.y1) * r1 + (cl.y3 - cl.y1) * r2;
-                    c.relocations++;
-                    // the phonon stays at the new point for the rest of the reference's drift:
-                    // up to the next boundary, or the flight's end if that comes first
-                    const double frozen = (double)(p.step + 1) * m.sim_time / (double)m.N - age;
-                    if (frozen < drift_time) { drift_time = frozen; }
-                    relocated = true;
-                    end_arg = drift_time;
-                    state = S_END;
-                } else if (cur_sensor != sensor0) {
-                    end_arg = drifted;
-                    state = S_END;
-                } else {
-                    state = S_NI;
-                }
+                passed = hit == HIT_PASSED;
+                state = !passed || ++collisions > MAX_COLLISIONS ? S_WALL : cur_sensor != sensor0 ? S_END : S_NI;
             }
         }
     };
@@ -660,32 +661,87 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
     // lanes whose drift ended in this iteration's impact search or collision.
     auto stage_end = [&]() {
         if (state == S_END) {
-            end_drift(end_arg);
+            end_drift();
             relocated = false;
         }
     };
-    // Scatter (lanes in S_SCAT), then the scattering-time draw (lanes in S_SCAT or S_TTS).
-    auto stage_scat = [&]() {
-        // One block for every lane of the stage: a scattering lane takes the scatter's draw
-        // and its next scattering-time draw from it, a lane that only draws a scattering time
-        // takes the first double.
-        double u_a = 0., u_b = 0.;
-        if (state == S_SCAT || state == S_TTS) { psim_urand2(&st, &u_a, &u_b); }
-        if (state == S_SCAT) {
-            c.scatters++;
-            scatter(m, p, relax, u_a, st);
-            u_a = u_b;
-            if (++events > PSIM_MAX_EVENTS_PER_STEP) {  // begin_event's stall bound
-                c.stalled++;
-                state = S_DEAD + FATE_STALLED * 8;
-            } else {
-                state = S_TTS;  // tts is 0 here, so begin_event would ask for a draw
+    // Every draw of the event loop: scatters (S_SCAT, ModelSimulator::scatter,
+    // modelSimulator.cpp:124-137), the scattering times after them or asked for alone (S_TTS), and
+    // reflections (S_WALL, BoundarySurface::handlePhonon, surface.cpp:32-44).  Lanes of all three
+    // share the first block and the new direction: a wave of the L-shape holds 55 scattering lanes
+    // and 11 reflecting ones per iteration, and reflections apart cost it a fifth of its instructions.
+    auto stage_draws = [&]() {
+        if (state == S_SCAT || state == S_TTS || state == S_WALL) {
+            const bool scat = state == S_SCAT, bounce = state == S_WALL && !passed;
+            const Sensor& sensor = m.sensors[cur_sensor];
+            double nx = 0., ny = 0., spec = 1.;
+            if (bounce) {
+                const Wall& w = m.walls[wall < 0 ? ~wall : wall];
+                nx = w.nx;
+                ny = w.ny;
+                spec = wall < 0 ? 0. : w.spec;
             }
-        }
-        if (state == S_TTS) {
-            relax_rates(m, cur_sensor, p, relax);
-            tts = SCALING_FACTOR * -psim_log(u_a) / (0. + relax[0] + relax[1] + relax[2]);
-            drift_setup();
+            psim_stream st = stream();
+            // The first block: a scattering lane takes the scatter's draw and its next scattering
+            // time's from it, a lane that only draws a scattering time its first double, a
+            // reflecting lane the draw that a specularity strictly between 0 and 1 is held
+            // against (at 0 the outcome is known: the block is passed over; a lane sent back by a
+            // transition and a mirror draw none).
+            double u_a = 1., u_b = 0.;
+            if (state != S_WALL || (spec != 1. && spec > 0.)) {
+                psim_urand2(&st, &u_a, &u_b);
+            } else if (spec != 1. && wall >= 0) {
+                ++st.block;
+            }
+            bool turn;  // takes a new direction
+            if (scat) {
+                const bool resampled = u_a <= rates.a;
+                if (resampled) { resample(m, sensor.material, sensor.scatter_table, p, st); }
+                turn = resampled ? u_a > rates.b : rates.impurity;
+            } else {
+                turn = bounce && spec != 1. && !(u_a < spec);
+            }
+            double tx = 0., ty = 0.;
+            if (turn) { new_direction(bounce, tx, ty, st); }
+            if (bounce) {
+                if (!turn) {  // specular
+                    tx = -p.dx * nx - p.dy * ny;
+                    ty = -p.dx * ny + p.dy * nx;
+                }
+                p.dx = nx * tx - ny * ty;
+                p.dy = ny * tx + nx * ty;
+            } else if (turn) {
+                p.dx = tx;
+                p.dy = ty;
+            }
+            if (state == S_WALL) {
+                if (!passed) { ++collisions; }
+                state = S_NI;
+                if (collisions > MAX_COLLISIONS) {  // Phonon::setRandPoint -> Triangle::getRandPoint
+                    double r1, r2;
+                    psim_urand2(&st, &r1, &r2);
+                    const psim_cell& cl = cold()->m.cells[p.cell];
+                    if (r1 + r2 > 1.) {
+                        r1 = 1 - r1;
+                        r2 = 1 - r2;
+                    }
+                    p.px = cl.x1 + (cl.x2 - cl.x1) * r1 + (cl.x3 - cl.x1) * r2;
+                    p.py = cl.y1 + (cl.y2 - cl.y1) * r1 + (cl.y3 - cl.y1) * r2;
+                    // the phonon stays at the new point for the rest of the reference's drift:
+                    // up to the next boundary, or the flight's end if that comes first
+                    const double frozen = boundary_time(p.step + 1) - age;
+                    if (frozen < drift_time) { drift_time = frozen; }
+                    relocated = true;
+                    drifted = drift_time;
+                    state = S_END;
+                }
+            } else if (scat && ++events > PSIM_MAX_EVENTS_PER_STEP) {  // begin_event's stall bound
+                state = S_DEAD + FATE_STALLED * 8;
+            } else {  // tts is 0 here after a scatter, so begin_event would ask for a draw
+                tts = scatter_time(sensor, p, scat ? u_b : u_a, rates);
+                drift_setup();
+            }
+            block = st.block;
         }
     };
 
@@ -701,9 +757,17 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
         const uint64_t m_fetch = __ballot(state == S_FETCH);
         if (m_fetch) { stage_fetch(m_fetch); }
         if (__ballot(state == S_NI)) { stage_ni(); }
-        if (__ballot(state == S_COLL)) { stage_coll(); }
+        const uint64_t m_coll = __ballot(state == S_COLL);
+        if (m_coll) {
+            wc.impacts += (uint32_t)__popcll(m_coll);
+            stage_coll();
+        }
         if (__ballot(state == S_END)) { stage_end(); }
-        if (__ballot(state == S_SCAT || state == S_TTS)) { stage_scat(); }
+        if (__ballot(state == S_SCAT || state == S_TTS || state == S_WALL)) {
+            wc.scatters += (uint32_t)__popcll(__ballot(state == S_SCAT));
+            stage_draws();
+            wc.relocations += (uint32_t)__popcll(__ballot(relocated));
+        }
 
         // Phonons that paused this iteration go to the next window's buffer, in slots the wave
         // has reserved; the dead leave.
@@ -720,44 +784,46 @@ transport_kernel(Model m, Pool pool, Lists lists, int32_t k0, int32_t k1, const 
             } else {
                 const int leader = __ffsll((unsigned long long)m_surv) - 1;
                 uint32_t base = 0;
-                if (lane == leader) { base = atomicAdd(lists.n_out, OUT_CLAIM); }
+                if (lane == leader) { base = atomicAdd(cold()->lists.n_out, OUT_CLAIM); }
                 base = __shfl(base, leader, WAVE);
                 k = rank < avail ? out_next + rank : base + (rank - avail);
                 out_next = base + (n_surv - avail);
                 out_end = base + OUT_CLAIM;
             }
             if (survive) {
-                const Live& O = lists.out;
-                O.pos[k] = make_double2(p.px, p.py);
-                O.dir[k] = make_double2(p.dx, p.dy);
-                O.fv[k] = make_double2(p.freq, p.vel);
-                O.at[k] = make_double2(age, tts);
-                O.r01[k] = make_double2(relax[0], relax[1]);
-                O.aux[k] = LiveAux{ relax[2], p.cell, cur_sensor };
-                O.tag[k] = LiveTag{ (uint32_t)p.bin | (p.pol == POL_TA ? META_TA : 0u) | (p.sign < 0 ? META_NEG : 0u)
-                                        | META_STARTED | (MULTI ? (st.c3 >> 8) << META_STREAM_SHIFT : 0u),
-                    slot, MULTI ? st.c2 : slot, p.step };
+                cold()->lists.out.rec[k] = LiveRec{ make_double2(p.px, p.py), make_double2(p.dx, p.dy), make_double2(p.freq, p.vel),
+                    make_double2(age, tts), make_double2(rates.a, rates.b),
+                    (p.pol == POL_TA ? META_TA : 0u) | (p.sign < 0 ? META_NEG : 0u) | (rates.impurity ? META_IMPURITY : 0u)
+                        | (MULTI ? (tag >> 8) << META_STREAM_SHIFT : 0u),
+                    slot, p.step, cur_sensor };
+                cold()->lists.out.cell[k] = make_uint2((uint32_t)p.cell, sid);
                 state = S_FETCH;
             }
         }
-        if (state >= S_DEAD) {
-            const int cause = (state - S_DEAD) / 8;
-            fate_write(fate, slot, cause == FATE_EXPIRED ? p.step - 1 : p.step, cause, p.px, p.py);
-            state = S_FETCH;
+        const uint64_t m_dead = __ballot(state >= S_DEAD);
+        if (m_dead) {
+            wc.absorbed += (uint32_t)__popcll(__ballot(state == S_DEAD + FATE_ABSORBED * 8));
+            wc.expired += (uint32_t)__popcll(__ballot(state == S_DEAD + FATE_EXPIRED * 8));
+            wc.stalled += (uint32_t)__popcll(__ballot(state == S_DEAD + FATE_STALLED * 8));
+            if (state >= S_DEAD) {
+                const int cause = (state - S_DEAD) / 8;
+                const Fate fate{ cold()->fate.step, cold()->fate.cause, cold()->fate.xy };
+                fate_write(fate, slot, cause == FATE_EXPIRED ? p.step - 1 : p.step, cause, p.px, p.py);
+                state = S_FETCH;
+            }
         }
     }
 
     // Reserved survivor slots the wave did not fill become holes.
-    for (uint32_t k = out_next + (uint32_t)lane; k < out_end; k += WAVE) { lists.out.aux[k].cell = -1; }
+    for (uint32_t k = out_next + (uint32_t)lane; k < out_end; k += WAVE) { cold()->lists.out.cell[k].x = ~0u; }
 
-    // Counters: wave sums, then one global atomic per wave and counter.
-    const uint32_t v[8] = { c.steps, c.scatters, c.impacts, c.relocations, c.absorbed, c.expired, c.tallies,
-        c.stalled };
+    // Counters: one global atomic per wave and counter.
+    const unsigned long long v[8] = { wave_sum64(n_steps), wc.scatters, wc.impacts, wc.relocations, wc.absorbed, wc.expired,
+        wave_sum64(n_tallies), wc.stalled };
     const int slots[8] = { PSIM_CNT_PHONON_STEPS, PSIM_CNT_SCATTERS, PSIM_CNT_IMPACTS, PSIM_CNT_RELOCATIONS,
         PSIM_CNT_ABSORBED, PSIM_CNT_EXPIRED, PSIM_CNT_TALLIES, PSIM_CNT_STALLED };
     for (int i = 0; i < 8; ++i) {
-        const unsigned long long sum = wave_sum64(v[i]);
-        if (lane == 0 && sum) { atomicAdd(&counters[slots[i]], sum); }
+        if (lane == 0 && v[i]) { atomicAdd(&cold()->counters[slots[i]], v[i]); }
     }
     if (WS) {  // the difference arrays summed over the window's steps, per sensor, into the partials
         __syncthreads();
@@ -803,7 +869,7 @@ __device__ __forceinline__ void sort_range(uint32_t n, uint32_t& lo, uint32_t& h
     hi = (uint32_t)std::min<uint64_t>(n, (uint64_t)lo + per);
 }
 
-__global__ void __launch_bounds__(SORT_BLOCK) cell_hist_kernel(const LiveAux* __restrict__ aux,
+__global__ void __launch_bounds__(SORT_BLOCK) cell_hist_kernel(const uint2* __restrict__ cell,
     const uint32_t* __restrict__ n_ptr, int shift, int n_keys, uint32_t* __restrict__ hist) {
     __shared__ uint32_t h[SORT_KEYS];
     for (int k = threadIdx.x; k < n_keys; k += SORT_BLOCK) { h[k] = 0; }
@@ -811,7 +877,7 @@ __global__ void __launch_bounds__(SORT_BLOCK) cell_hist_kernel(const LiveAux* __
     uint32_t lo, hi;
     sort_range(*n_ptr, lo, hi);
     for (uint32_t i = lo + threadIdx.x; i < hi; i += SORT_BLOCK) {
-        const int32_t cl = aux[i].cell;
+        const int32_t cl = (int32_t)cell[i].x;
         if (cl >= 0) { atomicAdd(&h[(uint32_t)cl >> shift], 1u); }
     }
     __syncthreads();
@@ -859,7 +925,7 @@ __global__ void __launch_bounds__(SORT_BLOCK) cell_scatter_kernel(Live src, Live
     uint32_t lo, hi;
     sort_range(*n_ptr, lo, hi);
     for (uint32_t i = lo + threadIdx.x; i < hi; i += SORT_BLOCK) {
-        const int32_t cl = src.aux[i].cell;
+        const int32_t cl = (int32_t)src.cell[i].x;
         if (cl >= 0) { atomicAdd(&cnt[(uint32_t)cl >> shift], 1u); }
     }
     __syncthreads();
@@ -869,17 +935,12 @@ __global__ void __launch_bounds__(SORT_BLOCK) cell_scatter_kernel(Live src, Live
     }
     __syncthreads();
     for (uint32_t i = lo + threadIdx.x; i < hi; i += SORT_BLOCK) {
-        const LiveAux ax = src.aux[i];
-        if (ax.cell < 0) { continue; }  // hole
-        const uint32_t key = (uint32_t)ax.cell >> shift;
+        const uint2 cs = src.cell[i];
+        if ((int32_t)cs.x < 0) { continue; }  // hole
+        const uint32_t key = cs.x >> shift;
         const uint32_t k = base[key] + atomicAdd(&cnt[key], 1u);
-        dst.pos[k] = src.pos[i];
-        dst.dir[k] = src.dir[i];
-        dst.fv[k] = src.fv[i];
-        dst.at[k] = src.at[i];
-        dst.r01[k] = src.r01[i];
-        dst.aux[k] = ax;
-        dst.tag[k] = src.tag[i];
+        dst.cell[k] = cs;
+        dst.rec[k] = src.rec[i];
     }
 }
 
@@ -1067,7 +1128,7 @@ void free_model(psim_gpu_ctx* c) {
 }
 
 void free_pool(psim_gpu_ctx* c) {
-    void* ps[] = { c->pool.pos, c->pool.dir, c->pool.fv, c->pool.aux, c->pool.ms };
+    void* ps[] = { c->pool.rec, c->pool.ms };
     for (void* p : ps) {
         if (p) { (void)hipFree(p); }
     }
@@ -1089,7 +1150,7 @@ void free_lists(psim_gpu_ctx* c) {
         if (p) { (void)hipFree(p); }
     }
     for (Live& L : c->live) {
-        void* ls[] = { L.pos, L.dir, L.fv, L.at, L.r01, L.aux, L.tag };
+        void* ls[] = { L.rec, L.cell };
         for (void* p : ls) {
             if (p) { (void)hipFree(p); }
         }
@@ -1214,12 +1275,9 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     if (c->pool_cap < n) {
         free_pool(c);
         const size_t cap = (size_t)std::max<int64_t>(n, 1);
-        c->pool.pos = dalloc<double2>(cap);
-        c->pool.dir = dalloc<double2>(cap);
-        c->pool.fv = dalloc<double2>(cap);
-        c->pool.aux = dalloc<PoolAux>(cap);
+        c->pool.rec = dalloc<PoolRec>(cap);
         c->pool.ms = dalloc<uint2>(cap);
-        if (!c->pool.pos || !c->pool.dir || !c->pool.fv || !c->pool.aux || !c->pool.ms) {
+        if (!c->pool.rec || !c->pool.ms) {
             free_pool(c);
             return fail(c, PSIM_E_DEVICE, "hipMalloc failed for the phonon pool");
         }
@@ -1259,14 +1317,9 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
         c->d_born_order = dalloc<uint32_t>(cap);
         bool ok = c->d_birth_key && c->d_born_order;
         for (Live& L : c->live) {
-            L.pos = dalloc<double2>(cap);
-            L.dir = dalloc<double2>(cap);
-            L.fv = dalloc<double2>(cap);
-            L.at = dalloc<double2>(cap);
-            L.r01 = dalloc<double2>(cap);
-            L.aux = dalloc<LiveAux>(cap);
-            L.tag = dalloc<LiveTag>(cap);
-            ok = ok && L.pos && L.dir && L.fv && L.at && L.r01 && L.aux && L.tag;
+            L.rec = dalloc<LiveRec>(cap);
+            L.cell = dalloc<uint2>(cap);
+            ok = ok && L.rec && L.cell;
         }
         if (!ok) {
             free_lists(c);
@@ -1339,9 +1392,9 @@ template <int NT, typename FT>
 void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Lists& lists, int32_t k0, int32_t k1,
     const Tally& t, const Fate& fate) {
     const dim3 g((unsigned)grid), b(NT);
+    const Args args{ c->m, c->pool, lists, t, fate, c->d_seed, c->d_counters, k0, k1 };
 #define PSIM_TRANSPORT(T, M, F)                                                                              \
-    hipLaunchKernelGGL((transport_kernel<T, M, NT, F>), g, b, lds, c->stream, c->m, c->pool, lists, k0, k1, c->d_seed, t, \
-        c->d_counters, fate)
+    hipLaunchKernelGGL((transport_kernel<T, M, NT, F>), g, b, lds, c->stream, args)
     // the untallied variant has no flux arrays: it is the same kernel for either flux type
     if (c->multi_stream) {
         if (tally == TALLY_NONE) {
@@ -1450,7 +1503,7 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
             const uint32_t* n_ptr = c->d_n_live + w + 1;
             const int sgrid = std::max(1, c->n_cu * 2);
             if ((rc = zero_fill(c, c->d_sort_keys, sizeof(uint32_t) * (size_t)n_keys)) != 0) { return rc; }
-            hipLaunchKernelGGL(cell_hist_kernel, dim3(sgrid), dim3(SORT_BLOCK), 0, c->stream, c->live[1].aux, n_ptr,
+            hipLaunchKernelGGL(cell_hist_kernel, dim3(sgrid), dim3(SORT_BLOCK), 0, c->stream, c->live[1].cell, n_ptr,
                 shift, n_keys, c->d_sort_keys);
             HIP_CHECK(c, hipGetLastError());
             hipLaunchKernelGGL(cell_scan_kernel, dim3(1), dim3(1024), 0, c->stream, c->d_sort_keys, n_keys,
@@ -1703,20 +1756,44 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
         m.field = d_;                                                                                    \
     } while (0)
     const size_t nb = (size_t)PSIM_NUM_FREQ_BINS;
-    PSIM_UPLOAD(cells, g->cells, g->n_cells);
-    PSIM_UPLOAD(edges, g->edges, (size_t)g->n_cells * 3);
-    PSIM_UPLOAD(subs, g->subs, g->n_subs);
-    std::vector<psim_sensor> sensors(g->sensors, g->sensors + g->n_sensors);
-    for (psim_sensor& se : sensors) {  // 0: the cap of one model with every sensor of the upload
-        if (se.flight_cap == 0) { se.flight_cap = psim_flight_cap(g->n_sensors); }
+    // The descriptors as the kernels read them (engine_device.hpp).
+    std::vector<Edge> edges((size_t)g->n_cells * 3);
+    std::vector<Wall> walls(edges.size() + (size_t)g->n_subs);
+    for (size_t i = 0; i < edges.size(); ++i) {
+        const psim_edge& e = g->edges[i];
+        edges[i] = Edge{ e.p1x, e.p1y, e.p2x, e.p2y, e.slope, e.intercept, rel_equals(e.p1x, e.p2x) ? 1 : 0, e.sub_begin,
+            e.n_trans + e.n_emit, 0 };
+        walls[i] = Wall{ e.nx, e.ny, e.spec, 0. };
     }
-    PSIM_UPLOAD(sensors, sensors.data(), g->n_sensors);
-    PSIM_UPLOAD(mats, t->materials, t->n_materials);
-    PSIM_UPLOAD(freq, t->freq, nb * t->n_materials);
-    PSIM_UPLOAD(vel_la, t->vel_la, nb * t->n_materials);
-    PSIM_UPLOAD(vel_ta, t->vel_ta, nb * t->n_materials);
-    PSIM_UPLOAD(cdf, t->cdf, nb * t->n_tables);
-    PSIM_UPLOAD(frac, t->la_frac, nb * t->n_tables);
+    std::vector<Sub> subs((size_t)g->n_subs);
+    for (size_t i = 0; i < subs.size(); ++i) {
+        const psim_subsurface& q = g->subs[i];
+        subs[i] = Sub{ q.p1x, q.p1y, q.p2x, q.p2y, q.kind, q.target,
+            q.target >= 0 && q.target < g->n_cells ? g->cells[q.target].sensor : 0, q.same_material, q.start, q.duration,
+            q.max_freq_la, q.max_freq_ta };
+        walls[edges.size() + i] = Wall{ q.nx, q.ny, q.spec, 0. };
+    }
+    std::vector<Sensor> sensors((size_t)g->n_sensors);
+    for (size_t i = 0; i < sensors.size(); ++i) {
+        const psim_sensor& q = g->sensors[i];
+        const psim_material& mt = t->materials[q.material];
+        // A vanishing temperature makes HBAR freq / tk so large that sinh overflows: the same with tk
+        // held where its reciprocal is finite.
+        double tk = q.t_init * BOLTZ;
+        if (tk >= 0. && tk < 1e-60) { tk = 1e-60; }
+        sensors[i] = Sensor{ mt.b_l, q.t3, mt.b_tn, q.t4, mt.b_tu, mt.b_i, mt.w, tk, 1. / tk, 0., q.material, q.scatter_table,
+            q.flight_cap ? q.flight_cap : psim_flight_cap(g->n_sensors), 0 };  // 0: the cap of one model with every sensor
+    }
+    std::vector<Bin> bins(nb * (size_t)t->n_materials);
+    for (size_t i = 0; i < bins.size(); ++i) {
+        bins[i] = Bin{ t->freq[i], t->vel_la[i], t->vel_ta[i], t->materials[i / nb].freq_width };
+    }
+    PSIM_UPLOAD(cells, g->cells, g->n_cells);
+    PSIM_UPLOAD(edges, edges.data(), edges.size());
+    PSIM_UPLOAD(walls, walls.data(), walls.size());
+    PSIM_UPLOAD(subs, subs.data(), subs.size());
+    PSIM_UPLOAD(sensors, sensors.data(), sensors.size());
+    PSIM_UPLOAD(bins, bins.data(), bins.size());
     PSIM_UPLOAD(sources, s->sources, s->n_sources);
     // Guide tables of the frequency search, when every cumulative table is non-decreasing (a
     // NaN fails the test too).
@@ -1724,22 +1801,23 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     for (int64_t i = 0; i + 1 < (int64_t)nb * t->n_tables && monotone; ++i) {
         if ((i + 1) % (int64_t)nb != 0 && !(t->cdf[i] <= t->cdf[i + 1])) { monotone = false; }
     }
-    if (monotone) {
-        std::vector<uint16_t> guide((size_t)(GUIDE + 1) * t->n_tables);
-        for (int k = 0; k < t->n_tables; ++k) {
-            const double* cdf = t->cdf + (size_t)k * nb;
-            int i = 0;
-            for (int g = 0; g <= GUIDE; ++g) {  // first index whose value exceeds g / GUIDE
-                const double x = (double)g / (double)GUIDE;
-                while (i < (int)nb && !(cdf[i] > x)) { ++i; }
-                guide[(size_t)k * (GUIDE + 1) + g] = (uint16_t)i;
-            }
+    m.guided = monotone ? 1 : 0;
+    std::vector<Table> tables((size_t)t->n_tables);
+    for (size_t k = 0; k < tables.size(); ++k) {
+        Table& tb = tables[k];
+        std::memcpy(tb.cdf, t->cdf + k * nb, sizeof tb.cdf);
+        std::memcpy(tb.frac, t->la_frac + k * nb, sizeof tb.frac);
+        std::memset(tb.guide, 0, sizeof tb.guide + sizeof tb.pad_);
+        int i = 0;
+        for (int g = 0; monotone && g <= GUIDE; ++g) {  // first index whose value exceeds g / GUIDE
+            const double x = (double)g / (double)GUIDE;
+            while (i < (int)nb && !(tb.cdf[i] > x)) { ++i; }
+            tb.guide[g] = (uint16_t)i;
         }
-        PSIM_UPLOAD(guide, guide.data(), guide.size());
-    } else {
-        m.guide = nullptr;
     }
+    PSIM_UPLOAD(tables, tables.data(), tables.size());
 #undef PSIM_UPLOAD
+    m.sub_walls = 3 * g->n_cells;
     m.n_sources = s->n_sources;
     m.n_sensors = g->n_sensors;
     m.full = p->full;
@@ -1751,6 +1829,7 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     m.sim_time = p->sim_time;
     m.step_time = p->step_time;
     m.t_eq = p->t_eq;
+    m.r_N = 1. / (double)p->num_measurements;
     c->m = m;
     c->params = *p;
     const int64_t SR = (int64_t)g->n_sensors * p->num_record;

@@ -33,29 +33,71 @@ constexpr int GUIDE = 2048;  // guide-table cells per frequency table (a power o
 enum : int { POL_LA = 0, POL_TA = 1 };
 enum : int { FATE_ABSORBED = 1, FATE_EXPIRED = 2, FATE_NOT_STARTED = 3, FATE_STALLED = 4 };
 
-// Phonon record word: bits 0-9 frequency bin, bit 10 TA, bit 11 negative sign, bit 12 started,
-// bits 16-31 random-stream index (the model's index in a batch, 0 otherwise).
-constexpr uint32_t META_BIN_MASK = 0x3ffu;
+// Phonon record word: bits 0-9 frequency bin (emission pool), bit 10 TA, bit 11 negative sign, bit 12
+// impurities scatter it (Rates::impurity), bits 16-31 random-stream index (the model's index in a batch, 0 otherwise).
 constexpr uint32_t META_TA = 1u << 10;
 constexpr uint32_t META_NEG = 1u << 11;
-constexpr uint32_t META_STARTED = 1u << 12;
+constexpr uint32_t META_IMPURITY = 1u << 12;
 constexpr int META_STREAM_SHIFT = 16;
+
+// One of a cell's three edges as the impact search and the surface stage read it: four 16-byte
+// loads.  `vert`: its ends have the same x up to rounding (rel_equals, tested once at upload).
+struct __attribute__((aligned(16))) Edge {
+    double p1x, p1y, p2x, p2y;
+    double slope, intercept;
+    int32_t vert;
+    int32_t sub_begin, n_sub;  // its sub-surfaces, transitions first
+    int32_t pad_;
+};
+
+// What a phonon reflects off: an edge's or a sub-surface's normal and specularity.
+struct __attribute__((aligned(16))) Wall {
+    double nx, ny, spec, pad_;
+};
+
+// A sub-surface: the line its containment test needs, then what a hit on it does.  The neighbour's
+// sensor stands beside the neighbour, so a transition needs no lookup of the cell entered.
+struct __attribute__((aligned(16))) Sub {
+    double p1x, p1y, p2x, p2y;
+    int32_t kind, target, target_sensor, same_material;
+    double start, duration;
+    double max_freq_la, max_freq_ta;
+};
+
+// What scattering in a sensor reads, its material's constants among it: one record, one address, so
+// the loads of a scattering phonon go out together instead of sensor first, material next.
+struct __attribute__((aligned(16))) Sensor {
+    double b_l, t3;
+    double b_tn, t4;
+    double b_tu, b_i;
+    double w, tk;  // tk = t_init x BOLTZ
+    double r_tk, pad0_;  // 1 / tk, rounded to nearest
+    int32_t material, scatter_table, flight_cap, pad_;
+};
+
+// A frequency bin of a material, with the material's bin width.
+struct __attribute__((aligned(16))) Bin {
+    double freq, vel_la, vel_ta, width;
+};
+
+// A frequency table: cumulative distribution, LA share of each bin and the start indices of the
+// frequency search.
+struct __attribute__((aligned(16))) Table {
+    double cdf[NBINS], frac[NBINS];
+    uint16_t guide[GUIDE + 1], pad_[7];
+};
 
 struct Model {
     const psim_cell* __restrict__ cells;
-    const psim_edge* __restrict__ edges;
-    const psim_subsurface* __restrict__ subs;
-    const psim_sensor* __restrict__ sensors;
-    const psim_material* __restrict__ mats;
-    const double* __restrict__ freq;
-    const double* __restrict__ vel_la;
-    const double* __restrict__ vel_ta;
-    const double* __restrict__ cdf;
-    const double* __restrict__ frac;
-    // [n_tables][GUIDE + 1] start indices of the frequency search, or null when some table is not
-    // monotone (then the bisection runs as written).
-    const uint16_t* __restrict__ guide;
+    const Edge* __restrict__ edges;  // [3 * n_cells]
+    const Wall* __restrict__ walls;  // [3 * n_cells] of the edges, then [n_subs] of the sub-surfaces
+    const Sub* __restrict__ subs;
+    const Sensor* __restrict__ sensors;
+    const Bin* __restrict__ bins;  // [n_materials][NBINS]
+    const Table* __restrict__ tables;
     const psim_source* __restrict__ sources;
+    int32_t guided;  // every table has its guide (else, some not monotone, the bisection runs as written)
+    int32_t sub_walls;  // 3 * n_cells
     int32_t n_sources;
     int32_t n_sensors;
     int32_t full;
@@ -69,23 +111,21 @@ struct Model {
     double sim_time;
     double step_time;
     double t_eq;
+    double r_N;  // 1 / N, rounded to nearest
 };
 
-// Birth time, cell (-1: never starts) and the cell's sensor of a pooled phonon.
-struct __attribute__((aligned(16))) PoolAux {
+// The emission pool, indexed by phonon id: a 64-byte record (one cache line half, four vector loads)
+// and the two words that are looked at apart.  A newborn phonon has no scattering time yet (0).
+struct __attribute__((aligned(16))) PoolRec {
+    double2 pos, dir;  // px py, dx dy
+    double2 fv;  // freq, vel
     double age;
-    int32_t cell;
+    int32_t cell;  // -1: never starts
     int32_t sensor;
 };
 
-// The emission pool, indexed by phonon id: five arrays of 8- and 16-byte records, so that a lane
-// moves a phonon in five vector loads and the kernels keep five pointers instead of twelve.  A
-// newborn phonon has no scattering time yet (0).
 struct Pool {
-    double2* __restrict__ pos;  // px, py
-    double2* __restrict__ dir;  // dx, dy
-    double2* __restrict__ fv;  // freq, vel
-    PoolAux* __restrict__ aux;
+    PoolRec* __restrict__ rec;
     uint2* __restrict__ ms;  // meta, id within the phonon's random stream (id - source id_base)
 };
 
@@ -95,52 +135,19 @@ struct Ph {
     int32_t step;
 };
 
-struct Line {
-    double p1x, p1y, p2x, p2y, slope, intercept, blx, bly, trx, try_;
-};
+// ---- division ---------------------------------------------------------------------------
+// Correctly rounded quotients by a divisor that several of them share (Markstein's method: with r
+// close enough to 1 / d, one remainder step in fused arithmetic rounds n / d correctly).  A full
+// division costs 11 FP64 instructions here; a quotient by a known reciprocal costs three.  For
+// finite n and d away from the ends of the exponent range, which callers see to.
+__device__ __forceinline__ double recip(double d) { return psim_recip(d); }
+__device__ __forceinline__ double div_by(double n, double d, double r) { return psim_div_by(n, d, r); }
+__device__ __forceinline__ double div_normal(double n, double d) { return PSIM_DIV(n, d); }
 
 // ---- geometry (psim/src/geometry.cpp) ------------------------------------------------
 
-__device__ __forceinline__ bool pt_eq(double ax, double ay, double bx, double by) {  // :34-39
-    const double dx = ax - bx;
-    const double dy = ay - by;
-    return dx * dx + dy * dy < GEOEPS * GEOEPS;
-}
-
 __device__ __forceinline__ double get_slope(double x1, double y1, double x2, double y2) {  // :325-327
     return (fabs(x1 - x2) < GEOEPS) ? 0. : (y1 - y2) / (x1 - x2);
-}
-
-__device__ __forceinline__ Line make_line(double x1, double y1, double x2, double y2) {  // :45-53, :267-280
-    Line l;
-    l.p1x = x1;
-    l.p1y = y1;
-    l.p2x = x2;
-    l.p2y = y2;
-    l.slope = get_slope(x1, y1, x2, y2);
-    l.intercept = y1 - l.slope * x1;
-    l.blx = (x2 <= x1) ? x2 : x1;
-    l.trx = (x2 <= x1) ? x1 : x2;
-    l.bly = (y2 <= y1) ? y2 : y1;
-    l.try_ = (y2 <= y1) ? y1 : y2;
-    return l;
-}
-
-// An edge's line from its endpoints, slope and intercept.  The bounding box is the min/max of the
-// endpoints, as the host builds it (the same values as the record's box), so it is not loaded.
-__device__ __forceinline__ Line edge_line(const psim_edge& e) {
-    Line l;
-    l.p1x = e.p1x;
-    l.p1y = e.p1y;
-    l.p2x = e.p2x;
-    l.p2y = e.p2y;
-    l.slope = e.slope;
-    l.intercept = e.intercept;
-    l.blx = (l.p2x <= l.p1x) ? l.p2x : l.p1x;
-    l.trx = (l.p2x <= l.p1x) ? l.p1x : l.p2x;
-    l.bly = (l.p2y <= l.p1y) ? l.p2y : l.p1y;
-    l.try_ = (l.p2y <= l.p1y) ? l.p1y : l.p2y;
-    return l;
 }
 
 // crossProduct of (p2 - p1) and (p - p1), :291-300, :311-313
@@ -154,45 +161,8 @@ __device__ __forceinline__ bool on_line(double x1, double y1, double x2, double 
     return fabs(line_cross(x1, y1, x2, y2, px, py)) < GEOEPS;
 }
 
-// doesSegmentCrossLine(l1, l2), :302-306
-__device__ __forceinline__ bool segment_crosses_line(const Line& l1, const Line& l2) {
-    const double c1 = line_cross(l1.p1x, l1.p1y, l1.p2x, l1.p2y, l2.p1x, l2.p1y);
-    const double c2 = line_cross(l1.p1x, l1.p1y, l1.p2x, l1.p2y, l2.p2x, l2.p2y);
-    return fabs(c1) < GEOEPS || fabs(c2) < GEOEPS || ((c1 < 0.) != (c2 < 0.));
-}
-
-__device__ __forceinline__ bool rel_equals(double a, double b) {  // :108-110
+__host__ __device__ __forceinline__ bool rel_equals(double a, double b) {  // :108-110
     return fabs(a - b) <= ((fabs(a) < fabs(b) ? fabs(b) : fabs(a)) * GEOEPS);
-}
-
-// Line::getIntersection(self = edge, other = path), :104-138 with Line::intersects :92-95
-// and boxesIntersect :282-289.
-__device__ __forceinline__ bool get_intersection(const Line& s, const Line& o, double& px, double& py) {
-    if (!(s.blx <= o.trx - GEOEPS && s.trx >= o.blx + GEOEPS && s.bly <= o.try_ - GEOEPS
-            && s.try_ >= o.bly + GEOEPS)) {
-        return false;
-    }
-    if (!segment_crosses_line(s, o) || !segment_crosses_line(o, s)) { return false; }
-    if (rel_equals(s.p1x, s.p2x)) {  // self vertical: handle_vert(self.p1, other.p1, other.p2)
-        if (rel_equals(o.p1x, o.p2x)) { return false; }
-        const double m = get_slope(o.p1x, o.p1y, o.p2x, o.p2y);
-        const double b = o.p1y - m * o.p1x;
-        px = s.p1x;
-        py = m * s.p1x + b;
-        return true;
-    }
-    if (rel_equals(o.p1x, o.p2x)) {  // other vertical: handle_vert(other.p1, self.p1, self.p2)
-        const double m = get_slope(s.p1x, s.p1y, s.p2x, s.p2y);
-        const double b = s.p1y - m * s.p1x;
-        px = o.p1x;
-        py = m * o.p1x + b;
-        return true;
-    }
-    if (rel_equals(s.slope, o.slope)) { return false; }
-    const double x = (o.intercept - s.intercept) / (s.slope - o.slope);
-    px = x;
-    py = s.slope * x + s.intercept;
-    return true;
 }
 
 // ---- phonon updates -------------------------------------------------------------------
@@ -204,16 +174,24 @@ __device__ __forceinline__ bool get_intersection(const Line& s, const Line& o, d
 // g = 0..GUIDE) that index lies in [guide[g], guide[g + 1]] for g = floor(rand * GUIDE), which a
 // short scan finds: one dependent load in place of ten.  Tables that are not non-decreasing
 // have no guide and run the bisection.
-__device__ __forceinline__ void freq_index(const double* __restrict__ cdf, const double* __restrict__ frac,
-    const uint16_t* __restrict__ guide, psim_stream& st, int& bin, int& pol) {
+__device__ __forceinline__ void freq_index(const Table& t, bool guided, psim_stream& st, int& bin, int& pol) {
+    const double* __restrict__ cdf = t.cdf;
     double rand, upol;  // the bisection's draw and the branch draw, one block
     psim_urand2(&st, &rand, &upol);
     int high;
-    if (guide) {
+    if (guided) {
         const int g = (int)(rand * (double)GUIDE);
-        int i = guide[g];
-        const int end = guide[g + 1];
-        while (i < end && !(rand < cdf[i])) { ++i; }
+        int i = t.guide[g];
+        const int end = t.guide[g + 1];
+        // the first two candidates in one round trip: a guide cell seldom spans more
+        const double c0 = cdf[i < NBINS ? i : NBINS - 1], c1 = cdf[i + 1 < NBINS ? i + 1 : NBINS - 1];
+        if (i < end && !(rand < c0)) {
+            ++i;
+            if (i < end && !(rand < c1)) {
+                ++i;
+                while (i < end && !(rand < cdf[i])) { ++i; }
+            }
+        }
         high = i < 1 ? 1 : (i > NBINS - 1 ? NBINS - 1 : i);
     } else {
         int low = 0;
@@ -229,161 +207,196 @@ __device__ __forceinline__ void freq_index(const double* __restrict__ cdf, const
         }
     }
     bin = high;
-    pol = (upol <= frac[high]) ? POL_LA : POL_TA;
-}
-
-__device__ __forceinline__ double bin_velocity(const Model& m, int mat, int bin, int pol) {  // material.cpp:82-84
-    return (pol == POL_LA) ? m.vel_la[mat * NBINS + bin] : m.vel_ta[mat * NBINS + bin];
+    pol = (upol <= t.frac[high]) ? POL_LA : POL_TA;
 }
 
 // SensorController::initialUpdate / scatterUpdate with Material::getFreq, sensorController.cpp:28-55,
 // material.cpp:77-80
 __device__ __forceinline__ void resample(const Model& m, int mat, int table, Ph& p, psim_stream& st) {
     int bin, pol;
-    freq_index(m.cdf + (int64_t)table * NBINS, m.frac + (int64_t)table * NBINS,
-        m.guide ? m.guide + (int64_t)table * (GUIDE + 1) : nullptr, st, bin, pol);
-    const psim_material& mt = m.mats[mat];
-    const double f0 = m.freq[mat * NBINS + bin];
-    p.freq = m.full ? f0 : f0 + (2. * psim_urand(&st) - 1.) * mt.freq_width / 2.;
+    freq_index(m.tables[table], m.guided != 0, st, bin, pol);
+    const Bin& bn = m.bins[mat * NBINS + bin];
+    const double f0 = bn.freq, vla = bn.vel_la, vta = bn.vel_ta, width = bn.width;
+    p.freq = m.full ? f0 : f0 + (2. * psim_urand(&st) - 1.) * width / 2.;
     p.bin = bin;
     p.pol = pol;
-    p.vel = bin_velocity(m, mat, bin, pol);
+    p.vel = (pol == POL_LA) ? vla : vta;  // material.cpp:82-84
 }
 
 __device__ __forceinline__ void set_rand_direction(Ph& p, psim_stream& st) {  // phonon.cpp:28-31
     double u1, u2;
     psim_urand2(&st, &u1, &u2);
     p.dx = 2. * u1 - 1.;
-    p.dy = sqrt(1. - p.dx * p.dx) * psim_cos2pi(u2);
+    p.dy = PSIM_SQRT(1. - p.dx * p.dx) * psim_cos2pi(u2);
 }
 
 __device__ __forceinline__ void redirect(double nx, double ny, Ph& p, psim_stream& st) {  // surface.cpp:23-30
     double rand, u2;
     psim_urand2(&st, &rand, &u2);
-    const double new_dx = sqrt(rand);
-    const double new_dy = sqrt(1. - rand) * psim_cos2pi(u2);
+    const double new_dx = PSIM_SQRT(rand);
+    const double new_dy = PSIM_SQRT(1. - rand) * psim_cos2pi(u2);
     p.dx = nx * new_dx - ny * new_dy;
     p.dy = ny * new_dx + nx * new_dy;
 }
 
-__device__ __forceinline__ void boundary_handle(double nx, double ny, double spec, Ph& p,
-    psim_stream& st) {  // surface.cpp:32-44
-    if (spec == 1. || psim_urand(&st) < spec) {
-        const double dx = p.dx, dy = p.dy;
-        const double new_dx = -dx * nx - dy * ny;
-        const double new_dy = -dx * ny + dy * nx;
-        p.dx = nx * new_dx - ny * new_dy;
-        p.dy = ny * new_dx + nx * new_dy;
-    } else {
-        redirect(nx, ny, p, st);
-    }
-}
+// Cell::handleSurfaceCollision -> CompositeSurface::handlePhonon (cell.cpp:103-108,
+// compositeSurface.cpp:47-66): the first edge the point of impact lies on, its first sub-surface the
+// point lies on, and what becomes of the phonon there.  Only the search and what moves the phonon
+// on stand here: a reflection waits for reflect(), which a wave runs together with its
+// scatters' draws and new directions.  `wall` is the index of the surface to reflect off, its
+// complement where a transition sends the phonon back (no specular reflection); `sensor` follows
+// the phonon into the cell it enters.
+enum : int { HIT_PASSED = 0, HIT_WALL = 1, HIT_ABSORBED = 2 };
 
-// Cell::handleSurfaceCollision -> CompositeSurface::handlePhonon and the surface handlers.
-__device__ __forceinline__ void handle_surface_collision(const Model& m, Ph& p, double poix, double poiy, psim_stream& st) {
-    const psim_edge* e3 = m.edges + 3 * p.cell;
-    for (int b = 0; b < 3; ++b) {
-        const psim_edge& e = e3[b];
-        if (!on_line(e.p1x, e.p1y, e.p2x, e.p2y, poix, poiy)) { continue; }
-        const int n_sub = e.n_trans + e.n_emit;
-        for (int i = 0; i < n_sub; ++i) {
-            const psim_subsurface& s = m.subs[e.sub_begin + i];
-            if (!on_line(s.p1x, s.p1y, s.p2x, s.p2y, poix, poiy)) { continue; }
-            if (s.kind == 0) {  // TransitionSurface::handlePhonon, surface.cpp:71-109
-                if (s.same_material) {
-                    p.cell = s.target;
-                } else {
-                    const double max_freq = (p.pol == POL_LA) ? s.max_freq_la : s.max_freq_ta;
-                    if (p.freq > max_freq) {
-                        redirect(s.nx, s.ny, p, st);
-                    } else {
-                        p.cell = s.target;
-                    }
-                }
-            } else {  // EmitSurface::handlePhonon, surface.cpp:61-65
-                const double phonon_time = (double)p.step * m.step_time;
-                if (phonon_time < s.start || phonon_time + m.step_time > s.start + s.duration) {
-                    boundary_handle(s.nx, s.ny, s.spec, p, st);
-                } else {
-                    p.cell = -1;
-                }
+__device__ __forceinline__ int surface_hit(const Model& m, Ph& p, int& sensor, int& wall) {
+    const Edge* e3 = m.edges + 3 * p.cell;
+    const Edge &e0 = e3[0], &e1 = e3[1], &e2 = e3[2];
+    const bool on0 = on_line(e0.p1x, e0.p1y, e0.p2x, e0.p2y, p.px, p.py);
+    const bool on1 = on_line(e1.p1x, e1.p1y, e1.p2x, e1.p2y, p.px, p.py);
+    const bool on2 = on_line(e2.p1x, e2.p1y, e2.p2x, e2.p2y, p.px, p.py);
+    if (!(on0 | on1 | on2)) { return HIT_PASSED; }
+    const int begin = on0 ? e0.sub_begin : on1 ? e1.sub_begin : e2.sub_begin;
+    const int n_sub = on0 ? e0.n_sub : on1 ? e1.n_sub : e2.n_sub;
+    wall = 3 * p.cell + (on0 ? 0 : on1 ? 1 : 2);
+    for (int i = begin; i < begin + n_sub; ++i) {
+        const Sub& s = m.subs[i];
+        if (!on_line(s.p1x, s.p1y, s.p2x, s.p2y, p.px, p.py)) { continue; }
+        wall = m.sub_walls + i;
+        if (s.kind == 0) {  // TransitionSurface::handlePhonon, surface.cpp:71-109
+            const double max_freq = (p.pol == POL_LA) ? s.max_freq_la : s.max_freq_ta;
+            if (!s.same_material && p.freq > max_freq) {
+                wall = ~wall;
+                return HIT_WALL;
             }
-            return;
+            p.cell = s.target;
+            sensor = s.target_sensor;
+            return HIT_PASSED;
         }
-        boundary_handle(e.nx, e.ny, e.spec, p, st);
-        return;
+        // EmitSurface::handlePhonon, surface.cpp:61-65
+        const double phonon_time = (double)p.step * m.step_time;
+        return phonon_time < s.start || phonon_time + m.step_time > s.start + s.duration ? HIT_WALL : HIT_ABSORBED;
     }
+    return HIT_WALL;
 }
-
-struct LaneCounters {
-    uint32_t steps, scatters, impacts, relocations, absorbed, expired, tallies, stalled;
-};
 
 // The geometric part of ModelSimulator::nextImpact (modelSimulator.cpp:87-117): the nearest edge
 // crossing of the path p -> p + v * time.  On a hit the phonon is moved to the point of impact
 // and the impact time is returned in out_time; the collision itself is handled separately
 // (modelSimulator.cpp:118).
-__device__ bool find_impact(const Model& m, Ph& p, double time, double& out_time, LaneCounters& c) {
+// Each edge runs Line::getIntersection (geometry.cpp:104-138: boxesIntersect :282-289,
+// doesSegmentCrossLine :302-306 both ways, then the point) with the reference's operations and
+// roundings; what depends on the path alone (its box, slope, direction, the reciprocals of its
+// velocity) is computed once, and differences that only change sign are shared (negation is exact).
+__device__ __forceinline__ bool find_impact(const Model& m, Ph& p, double time, double& out_time) {
     const double vx = p.dx * p.vel;
     const double vy = p.dy * p.vel;
     const double sx = p.px, sy = p.py;
     const double ex = p.px + time * vx, ey = p.py + time * vy;
-    if (pt_eq(sx, sy, ex, ey)) { return false; }
-    const Line path = make_line(sx, sy, ex, ey);
-    const psim_edge* e3 = m.edges + 3 * p.cell;
+    const double ddx = sx - ex, ddy = sy - ey;
+    if (ddx * ddx + ddy * ddy < GEOEPS * GEOEPS) { return false; }  // pt_eq(start, end)
+    const double os = (fabs(ddx) < GEOEPS) ? 0. : div_normal(ddy, ddx);  // the path's slope and intercept
+    const double oi = sy - os * sx;
+    const bool o_vert = rel_equals(sx, ex);
+    // the path's box, drawn in by GEOEPS
+    const double hix = ((ex <= sx) ? sx : ex) - GEOEPS, lox = ((ex <= sx) ? ex : sx) + GEOEPS;
+    const double hiy = ((ey <= sy) ? sy : ey) - GEOEPS, loy = ((ey <= sy) ? ey : sy) + GEOEPS;
+    const bool move_x = vx > VELOCITY_EPS || vx < -VELOCITY_EPS;
+    const bool move_y = vy > VELOCITY_EPS || vy < -VELOCITY_EPS;
+    const double rvx = recip(vx), rvy = recip(vy);  // used where move_x / move_y
+    const Edge* e3 = m.edges + 3 * p.cell;
     bool hit = false;
     double ix = 0., iy = 0.;
+    #pragma unroll
     for (int b = 0; b < 3; ++b) {
-        const Line l = edge_line(e3[b]);
+        const Edge& s = e3[b];
+        const double p1x = s.p1x, p1y = s.p1y, p2x = s.p2x, p2y = s.p2y;
+        const bool box = ((p1x <= hix) | (p2x <= hix)) & ((p1x >= lox) | (p2x >= lox)) & ((p1y <= hiy) | (p2y <= hiy))
+                         & ((p1y >= loy) | (p2y >= loy));
+        const double ax = p2x - p1x, ay = p2y - p1y;
+        const double b1x = sx - p1x, b1y = sy - p1y, b2x = ex - p1x, b2y = ey - p1y;
+        const double c1 = ax * b1y - b1x * ay, c2 = ax * b2y - b2x * ay;  // path ends against the edge's line
+        const double f2x = p2x - sx, f2y = p2y - sy;
+        const double d1 = ddx * b1y - b1x * ddy, d2 = f2x * ddy - ddx * f2y;  // edge ends against the path's
+        const bool cross = ((fabs(c1) < GEOEPS) | (fabs(c2) < GEOEPS) | ((c1 < 0.) != (c2 < 0.)))
+                           & ((fabs(d1) < GEOEPS) | (fabs(d2) < GEOEPS) | ((d1 < 0.) != (d2 < 0.)));
+        if (!(box & cross)) { continue; }
+        const double ss = s.slope, si = s.intercept;
+        const bool s_vert = s.vert != 0;
         double qx, qy;
-        if (get_intersection(l, path, qx, qy) && !pt_eq(qx, qy, sx, sy)) {
-            const double tx = (vx > VELOCITY_EPS || vx < -VELOCITY_EPS) ? (qx - sx) / vx : time;
-            const double ty = (vy > VELOCITY_EPS || vy < -VELOCITY_EPS) ? (qy - sy) / vy : time;
-            const double it = (tx <= ty) ? tx : ty;
-            if (it <= time) {
-                time = it;
-                ix = qx;
-                iy = qy;
-                hit = true;
-            }
+        if (o_vert && !s_vert) {  // the path vertical
+            const double mm = get_slope(p1x, p1y, p2x, p2y);
+            qx = sx;
+            qy = mm * sx + (p1y - mm * p1x);
+        } else {
+            if (s_vert ? o_vert : rel_equals(ss, os)) { continue; }
+            qx = s_vert ? p1x : div_normal(oi - si, ss - os);
+            qy = (s_vert ? os : ss) * qx + (s_vert ? oi : si);
+        }
+        const double gx = qx - sx, gy = qy - sy;
+        if (gx * gx + gy * gy < GEOEPS * GEOEPS) { continue; }  // pt_eq(point, start)
+        const double tx = move_x ? div_by(gx, vx, rvx) : time;
+        const double ty = move_y ? div_by(gy, vy, rvy) : time;
+        const double it = (tx <= ty) ? tx : ty;
+        if (it <= time) {
+            time = it;
+            ix = qx;
+            iy = qy;
+            hit = true;
         }
     }
     if (hit) {
         p.px = ix;
         p.py = iy;
-        c.impacts++;
         out_time = time;
     }
     return hit;
 }
 
-// Material::relaxRates at the sensor temperature, material.cpp:54-56, 207-239
-__device__ __forceinline__ void relax_rates(const Model& m, int sensor, const Ph& p, double* r) {
-    const psim_sensor& s = m.sensors[sensor];
-    const psim_material& mt = m.mats[s.material];
+// Material::relaxRates at the sensor temperature (material.cpp:54-56, 207-239) and what a scatter
+// and a scattering time need of them: the shares of the total rate up to which a scatter
+// resamples (a, (r0 + r1) / total) and keeps its direction (b, r0 / total), whether impurities
+// scatter at all, and the time to the next scatter, SCALING_FACTOR * -log(u) / total
+// (modelSimulator.cpp:124-137, 158-162).  The three quotients share their divisor.
+struct Rates {
+    double a, b;
+    bool impurity;
+};
+
+__device__ __forceinline__ double scatter_time(const Sensor& s, const Ph& p, double u, Rates& r) {
     const double freq = p.freq;
+    double r0, r1;
     if (p.pol == POL_LA) {
-        r[0] = mt.b_l * freq * freq * s.t3;
-        r[1] = mt.b_l * freq * freq * s.t3;
+        r0 = s.b_l * freq * freq * s.t3;
+        r1 = r0;
     } else {
-        r[0] = (freq < mt.w) ? mt.b_tn * freq * s.t4 : 0.;
-        r[1] = (freq >= mt.w) ? mt.b_tu * freq * freq / psim_sinh(HBAR * freq / (s.t_init * BOLTZ)) : 0.;
+        r0 = (freq < s.w) ? s.b_tn * freq * s.t4 : 0.;
+        r1 = (freq >= s.w) ? s.b_tu * freq * freq / psim_sinh(div_by(HBAR * freq, s.tk, s.r_tk)) : 0.;
     }
-    r[2] = mt.b_i * psim_pow4(freq);
+    const double r2 = s.b_i * psim_pow4(freq);
+    const double total = 0. + r0 + r1 + r2;
+    const double n = SCALING_FACTOR * -psim_log(u);
+    r.impurity = r2 > 0.;
+    if (u > 0. && total > 1e-100 && total < 1e100) {
+        const double rt = recip(total);
+        r.a = div_by(r0 + r1, total, rt);
+        r.b = div_by(r0, total, rt);
+        return div_by(n, total, rt);
+    }
+    r.a = (r0 + r1) / total;
+    r.b = r0 / total;
+    return n / total;
 }
 
-// ModelSimulator::scatter, modelSimulator.cpp:124-137, with its draw `rand` taken by the caller
-// (together with the next scattering-time draw, one block).
-// The new direction of an Umklapp scatter (after the resample) and of an impurity scatter is one
-// code path, so a wave holding both runs it once.
-__device__ __forceinline__ void scatter(const Model& m, Ph& p, const double* r, double rand, psim_stream& st) {
-    const double tau_inv = 0. + r[0] + r[1] + r[2];
-    const bool resampled = rand <= (r[0] + r[1]) / tau_inv;
-    if (resampled) {
-        const psim_sensor& s = m.sensors[m.cells[p.cell].sensor];
-        resample(m, s.material, s.scatter_table, p, st);
-    }
-    if (resampled ? rand > r[0] / tau_inv : r[2] > 0.) { set_rand_direction(p, st); }
+// A new direction: Surface::redirectPhonon off a wall (surface.cpp:23-30), before its rotation to
+// the wall's normal, or Phonon::setRandDirection (phonon.cpp:28-31).  Both take the next block and
+// end in sqrt(..) cos(2 pi u); one pass serves lanes of either kind.
+__device__ __forceinline__ void new_direction(bool off_wall, double& dx, double& dy, psim_stream& st) {
+    double u1, u2;
+    psim_urand2(&st, &u1, &u2);
+    const double along = 2. * u1 - 1.;
+    const double c = psim_cos2pi(u2);
+    dy = PSIM_SQRT(1. - (off_wall ? u1 : along * along)) * c;
+    dx = off_wall ? PSIM_SQRT(u1) : along;
 }
 
 }  // namespace psim_dev

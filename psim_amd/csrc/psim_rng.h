@@ -64,6 +64,11 @@ PSIM_QUAL psim_u32x4 psim_philox_round(psim_u32x4 c, uint32_t k0, uint32_t k1) {
 /* Philox4x32 with 10 rounds; the key is bumped by the Weyl constants between
  * rounds. */
 PSIM_QUAL psim_u32x4 psim_philox4x32_10(psim_u32x4 c, uint32_t k0, uint32_t k1) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* unrolled; the round keys are added up here, not kept in scalar registers across the caller's loop */
+    asm volatile("" : "+s"(k0), "+s"(k1));
+#pragma unroll
+#endif
     for (int i = 0; i < 9; ++i) {
         c = psim_philox_round(c, k0, k1);
         k0 += PSIM_PHILOX_W0;
@@ -74,8 +79,13 @@ PSIM_QUAL psim_u32x4 psim_philox4x32_10(psim_u32x4 c, uint32_t k0, uint32_t k1) 
 
 /* 53 high bits of (hi:lo) scaled into [0, 1). */
 PSIM_QUAL double psim_u01_from_pair(uint32_t hi, uint32_t lo) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* both terms and their sum are exact */
+    return __builtin_fma((double)hi, 0x1.0p-32, (double)(lo >> 11) * 0x1.0p-53);
+#else
     const uint64_t bits = ((uint64_t)hi << 32) | (uint64_t)lo;
     return (double)(bits >> 11) * 0x1.0p-53;
+#endif
 }
 
 /* A stream of uniform doubles in [0, 1): one Philox block per draw. */
