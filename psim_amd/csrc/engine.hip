@@ -47,6 +47,14 @@ constexpr int GLOBAL_TALLY_STEPS = 16;  // fewer LDS-tallied steps per window th
 // above).
 constexpr int64_t LDS_MIN_PHONONS_PER_SENSOR = 30000;
 constexpr uint32_t QUEUE_CLAIM = 32;  // work-queue items a wave claims per atomic
+// A run of fewer phonons than the chip has lanes is as long as its longest-lived phonon: each event
+// waits for the one before.  An iteration costs a wave every stage that any of its lanes is in, so
+// such a run spreads over this many waves per CU (as many as fit with the untallied variant's
+// registers), each carrying fewer phonons, and a wave claims no phonon ahead of need.  Bar of 1e5
+// phonons: 64 / 32 / 16 / 8 / 1 lanes 13.2 / 12.1 / 11.6 / 12.2 / 16.5 ms (24 by this rule); of 5000:
+// 4.0 / 3.6 / 3.4 / 2.7 / 2.6 ms (2 by this rule).  At 1e6 phonons fewer lanes lose (64 / 48 / 32:
+// 35.9 / 36.3 / 40.6 ms), and there claims of one item cost the atomics' latency (lshape 159 -> 231 ms).
+constexpr int SPREAD_WAVES_PER_CU = 16;
 constexpr uint32_t OUT_CLAIM = 64;  // survivor slots a wave reserves per atomic
 
 // Tallies of a launch window.  A boundary a flight passes is recorded as part of a segment: the
@@ -336,6 +344,8 @@ struct Args {
     const uint64_t* __restrict__ seed_p;
     unsigned long long* __restrict__ counters;
     int32_t k0, k1;
+    int32_t lanes;  // lanes of a wave that carry phonons (64 but for small runs)
+    uint32_t claim;  // work-queue items a wave claims per atomic
 };
 
 typedef const __attribute__((address_space(4))) Args* ArgsPtr;
@@ -379,7 +389,7 @@ transport_kernel(Args args) {
     const int64_t b0 = args.lists.born_offset[k0];
     const int64_t n_items = n_live + (int64_t)args.lists.born_offset[k1] - b0;
 
-    int state = S_FETCH;
+    int state = lane < args.lanes ? S_FETCH : S_EXIT;
     uint32_t slot = 0;
     Ph p;
     p.px = p.py = p.dx = p.dy = p.freq = p.vel = 0.;
@@ -417,7 +427,7 @@ transport_kernel(Args args) {
         return c2 < m.N ? c2 : m.N;
     };
     // Work-queue items the wave has claimed but not handed out yet (wave-uniform): a refill takes
-    // them in order and claims QUEUE_CLAIM more with one atomic when they run out.
+    // them in order and claims args.claim more with one atomic when they run out.
     uint32_t res_next = 0, res_end = 0;
     uint32_t out_next = 0, out_end = 0;  // survivor slots reserved by the wave, not filled yet
 
@@ -562,7 +572,7 @@ transport_kernel(Args args) {
             res_next += n_fetch;
         } else {
             const uint32_t need = n_fetch - avail;
-            const uint32_t take = need > QUEUE_CLAIM ? need : QUEUE_CLAIM;
+            const uint32_t take = need > args.claim ? need : args.claim;
             const int leader = __ffsll((unsigned long long)m_fetch) - 1;
             uint32_t base = 0;
             if (lane == leader) { base = atomicAdd(cold()->lists.queue + cold()->lists.window, take); }
@@ -1256,7 +1266,7 @@ std::vector<std::pair<int64_t, int64_t>> plan_windows(int64_t N, int64_t adj, in
 // Launch plan of one run of the uploaded model.
 struct RunPlan {
     int64_t n = 0, N = 0, R = 0, blocks_needed = 0, steps_need = 0, WS = 0;
-    int S = 0, grid = 1;
+    int S = 0, grid = 1, lanes = WAVE;
     int32_t W = 0;
     bool global_tally = false;
     std::vector<std::pair<int64_t, int64_t>> windows;
@@ -1299,12 +1309,15 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     }
     const int64_t blocks_needed = (n + BLOCK - 1) / BLOCK;  // emission and birth sort: one thread per phonon
     const int tb = c->tally_fp32 ? 256 : c->block;  // transport threads per block (FP32 tallies: 256)
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((n + tb - 1) / tb, (int64_t)c->n_cu * c->blocks_per_cu));
+    const int64_t max_blocks = (int64_t)c->n_cu * c->blocks_per_cu, block_waves = tb / WAVE;
+    const int64_t spread = std::min<int64_t>((int64_t)c->n_cu * SPREAD_WAVES_PER_CU, max_blocks * block_waves);
+    const int lanes = (int)std::max<int64_t>(1, std::min<int64_t>(WAVE, (n + spread - 1) / spread));
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((n + lanes * block_waves - 1) / (lanes * block_waves), max_blocks));
     // Each lane counts its phonon-steps, tallies and events in 32 bits until the launch ends (the
     // wave sums are 64-bit).  The work queue spreads the phonons evenly over the lanes, so a lane
     // carries about n * N / lanes phonon-steps at most; runs where that average comes within a
     // factor of 2 of 2^32 are refused rather than risk a wrapped counter.
-    const double lane_share = (double)n * (double)P.num_measurements / ((double)grid * tb);
+    const double lane_share = (double)n * (double)P.num_measurements / ((double)grid * block_waves * lanes);
     if (lane_share >= 2147483648.0) {
         return fail(c, PSIM_E_INVALID, "run too large: phonons x measurement steps per lane exceeds 2^31");
     }
@@ -1371,6 +1384,7 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     plan.S = S;
     plan.blocks_needed = blocks_needed;
     plan.grid = grid;
+    plan.lanes = lanes;
     plan.steps_need = steps_need;
     plan.WS = WS;
     plan.W = W;
@@ -1389,10 +1403,8 @@ int zero_fill(psim_gpu_ctx* c, void* p, size_t bytes) {
 
 // One transport launch of the variant for this tally path, stream layout, block size and flux type.
 template <int NT, typename FT>
-void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Lists& lists, int32_t k0, int32_t k1,
-    const Tally& t, const Fate& fate) {
+void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Args& args) {
     const dim3 g((unsigned)grid), b(NT);
-    const Args args{ c->m, c->pool, lists, t, fate, c->d_seed, c->d_counters, k0, k1 };
 #define PSIM_TRANSPORT(T, M, F)                                                                              \
     hipLaunchKernelGGL((transport_kernel<T, M, NT, F>), g, b, lds, c->stream, args)
     // the untallied variant has no flux arrays: it is the same kernel for either flux type
@@ -1415,16 +1427,15 @@ void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const
 }
 
 // The FP32 tally precision runs 256-thread blocks only (one more set of kernels, not three).
-void launch_transport(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Lists& lists, int32_t k0, int32_t k1,
-    const Tally& t, const Fate& fate) {
+void launch_transport(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Args& args) {
     if (c->tally_fp32) {
-        launch_transport_nt<256, float>(c, tally, grid, lds, lists, k0, k1, t, fate);
+        launch_transport_nt<256, float>(c, tally, grid, lds, args);
     } else if (c->block == 128) {
-        launch_transport_nt<128, double>(c, tally, grid, lds, lists, k0, k1, t, fate);
+        launch_transport_nt<128, double>(c, tally, grid, lds, args);
     } else if (c->block == 512) {
-        launch_transport_nt<512, double>(c, tally, grid, lds, lists, k0, k1, t, fate);
+        launch_transport_nt<512, double>(c, tally, grid, lds, args);
     } else {
-        launch_transport_nt<256, double>(c, tally, grid, lds, lists, k0, k1, t, fate);
+        launch_transport_nt<256, double>(c, tally, grid, lds, args);
     }
 }
 
@@ -1476,8 +1487,9 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
         // (W + 1) rows per sensor of a count and two flux values
         const size_t lds = (rec && !global_tally) ? (size_t)(WS + S) * (c->tally_fp32 ? 12 : 20) : 0;
         if (eager) { HIP_CHECK(c, hipEventRecord(c->ev[1], c->stream)); }
-        launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, lists,
-            (int32_t)k0, (int32_t)k1, t, fate);
+        const Args args{ c->m, c->pool, lists, t, fate, c->d_seed, c->d_counters, (int32_t)k0, (int32_t)k1, plan.lanes,
+            plan.lanes < WAVE ? 1u : QUEUE_CLAIM };
+        launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, args);
         HIP_CHECK(c, hipGetLastError());
         if (eager) { HIP_CHECK(c, hipEventRecord(c->ev[2], c->stream)); }
         if (rec && !global_tally) {
