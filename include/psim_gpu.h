@@ -225,7 +225,8 @@ int psim_gpu_last_timing(const psim_gpu_ctx* ctx, double* step_kernel_ms, int64_
 
 /* Engine tuning: measurement steps per transport launch (0 = automatic).  No length changes a
  * result.  By default a recording launch (LDS tallies) is as long as the model's flight cap
- * (psim_flight_cap), so it holds whole flights; a window that does not line up with the caps lets
+ * (psim_flight_cap), so it holds whole flights, or, in a run of enough phonons, as long as several
+ * caps that fit a CU's whole LDS; a window that does not line up with the caps lets
  * flights pass its end, and their boundaries past it are tallied in HBM (same sums, slower). */
 int psim_gpu_set_window(psim_gpu_ctx* ctx, int32_t steps_per_launch);
 
@@ -253,8 +254,8 @@ int psim_gpu_set_tally_mode(psim_gpu_ctx* ctx, int32_t mode);
  * Sensor::updateHeatParams does (psim/src/sensor.cpp:43-52).  FP32_KAHAN keeps the LDS window
  * difference arrays and the HBM ones in FP32 (FP32 atomics), sums the window partials along the
  * steps and across blocks with Kahan compensation in FP32, and returns each tally as
- * sum - compensation in the same double arrays; integer counts are unaffected.  The launch plan
- * and trajectories are those of FP64 (its transport blocks are 256 threads), so a run of each on
+ * sum - compensation in the same double arrays; integer counts are unaffected.  The trajectories
+ * are those of FP64 (its launches are the narrow 256-thread ones), so a run of each on
  * one seed shows the error of the FP32 tallies against FP64.  No counterpart in the reference. */
 #define PSIM_TALLY_FP64 0
 #define PSIM_TALLY_FP32_KAHAN 1

@@ -40,12 +40,19 @@ namespace {
 constexpr int BLOCK = 256;
 constexpr int WAVE = 64;
 constexpr int LDS_TALLY_BYTES = 48 * 1024;  // budget for one block's [W][S] window tally
+constexpr int LDS_WIDE_BYTES = 160 * 1024;  // the same where one block has a CU to itself
 constexpr int GLOBAL_TALLY_STEPS = 16;  // fewer LDS-tallied steps per window than this: HBM tallies
 // Fewer phonons per sensor than this: global atomics too.  Small runs lose more to the many short
 // LDS windows (launches, reductions, sorts) than HBM atomics lose to contention, large ones the
 // reverse (measured at 1e4 and 1e5 phonons per sensor: 1.8-3x faster in HBM below, 2.7x slower
 // above).
 constexpr int64_t LDS_MIN_PHONONS_PER_SENSOR = 30000;
+// The same with wide windows (wide_window_for) of at least WIDE_LDS_STEPS steps, of which a run has few:
+// film of 3e5 phonons (10000 per sensor) 14.2 ms in LDS, 30.4 in HBM; L-shape of 3e5 (7500) periodic
+// 18.1 against 26.3, steady state 17.5 against 17.6; with 69-step windows (bar of 100 sensors) LDS
+// still loses at 10000 per sensor, 42.3 against 34.5.
+constexpr int32_t WIDE_LDS_STEPS = 128;
+constexpr int64_t WIDE_MIN_PHONONS_PER_SENSOR = 7500;
 constexpr uint32_t QUEUE_CLAIM = 32;  // work-queue items a wave claims per atomic
 // A run of fewer phonons than the chip has lanes is as long as its longest-lived phonon: each event
 // waits for the one before.  An iteration costs a wave every stage that any of its lanes is in, so
@@ -1068,6 +1075,7 @@ struct psim_gpu_ctx {
     std::vector<void*> model_allocs;
     int32_t n_sensors = 0;
     int32_t n_cells = 0;
+    int32_t flight_cap = 0;  // of every sensor (0: they differ)
     // run buffers
     Pool pool{};
     int64_t pool_cap = 0;
@@ -1230,6 +1238,25 @@ int32_t record_window_for(const psim_gpu_ctx* c) {
     return (int32_t)std::min<int64_t>(c->window > 0 ? c->window : 128, by_lds);
 }
 
+// Wide recording windows: one block of WIDE_BLOCK threads per CU whose tallies take the CU's whole
+// LDS, and windows of as many flight caps as then fit (0: none).  Every window ends with a tail in
+// which the last phonons finish, a sort and a reduction, so fewer windows run faster, and one block's
+// tallies per CU instead of up to eight are a quarter of the partials.  128 registers leave 16 waves
+// on the CU as four blocks of 256 would, which the smaller budget's tallies would not.  For runs that
+// fill those blocks' lanes and whose models share a flight cap that fits twice; launch shapes set by
+// the caller are kept to.  Film of 3e6 phonons (240 steps a window, was 80) 70.7 ms, with 768 threads
+// 77.4, with the narrow windows 88.1; periodic L-shape of 1.6e6 (180, was 60) 53.0 / 55.5 / 66.0 ms.
+constexpr int WIDE_BLOCK = 1024;
+int32_t wide_window_for(const psim_gpu_ctx* c) {
+    if (c->window > 0 || c->block != 256 || c->tally_fp32 || c->flight_cap <= 0
+        || c->params.total_phonons < (int64_t)c->n_cu * WIDE_BLOCK) {
+        return 0;
+    }
+    const int64_t rows = LDS_WIDE_BYTES / (20 * (int64_t)std::max(1, c->n_sensors)) - 1;
+    const int32_t caps = (int32_t)(rows / c->flight_cap);
+    return caps >= 2 ? caps * c->flight_cap : 0;
+}
+
 int32_t free_window_for(const psim_gpu_ctx* c) { return c->window > 0 ? c->window : DEFAULT_FREE_WINDOW; }
 
 // Tally path of a run: LDS window partials for runs with enough phonons per sensor when enough
@@ -1240,6 +1267,7 @@ bool use_global_tally(const psim_gpu_ctx* c) {
     const int64_t lds_steps = LDS_TALLY_BYTES / (20 * sensors) - 1;
     if (c->tally_mode == PSIM_TALLY_HBM || lds_steps < 1) { return true; }
     if (c->tally_mode == PSIM_TALLY_LDS) { return false; }
+    if (wide_window_for(c) >= WIDE_LDS_STEPS) { return c->params.total_phonons < WIDE_MIN_PHONONS_PER_SENSOR * sensors; }
     return lds_steps < GLOBAL_TALLY_STEPS || c->params.total_phonons < LDS_MIN_PHONONS_PER_SENSOR * sensors;
 }
 
@@ -1267,6 +1295,8 @@ std::vector<std::pair<int64_t, int64_t>> plan_windows(int64_t N, int64_t adj, in
 struct RunPlan {
     int64_t n = 0, N = 0, R = 0, blocks_needed = 0, steps_need = 0, WS = 0;
     int S = 0, grid = 1, lanes = WAVE;
+    int rec_grid = 1;  // blocks of a recording launch with LDS tallies
+    bool wide = false;
     int32_t W = 0;
     bool global_tally = false;
     std::vector<std::pair<int64_t, int64_t>> windows;
@@ -1322,7 +1352,7 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
         return fail(c, PSIM_E_INVALID, "run too large: phonons x measurement steps per lane exceeds 2^31");
     }
     // A live buffer holds every phonon plus the survivor slots the waves may reserve but not fill.
-    const int64_t live_need = n + (int64_t)OUT_CLAIM * grid * (tb / WAVE);
+    const int64_t live_need = n + (int64_t)OUT_CLAIM * std::max<int64_t>(grid * block_waves, (int64_t)c->n_cu * (WIDE_BLOCK / WAVE));
     if (c->list_cap < live_need) {
         free_lists(c);
         const size_t cap = (size_t)std::max<int64_t>(live_need, 1);
@@ -1342,7 +1372,9 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
         c->gen++;
     }
     const bool global_tally = use_global_tally(c);
-    const int32_t W = global_tally ? free_window_for(c) : record_window_for(c);
+    const int32_t wide = global_tally ? 0 : wide_window_for(c);
+    const int32_t W = global_tally ? free_window_for(c) : wide ? wide : record_window_for(c);
+    const int rec_grid = wide ? c->n_cu : grid;
     const int64_t N = P.num_measurements;
     const auto windows = plan_windows(N, P.step_adjustment, free_window_for(c), W);
     const int64_t n_windows = (int64_t)windows.size();
@@ -1363,9 +1395,9 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
         c->gen++;
     }
     const int64_t WS = global_tally ? 0 : (int64_t)W * S;
-    if (c->partial_cap < grid * WS) {
+    if (c->partial_cap < rec_grid * WS) {
         free_partials(c);
-        const size_t cap = (size_t)(grid * WS);
+        const size_t cap = (size_t)(rec_grid * WS);
         c->d_pcnt = dalloc<int32_t>(cap);
         c->d_pfx = dalloc<double>(cap);
         c->d_pfy = dalloc<double>(cap);
@@ -1385,6 +1417,8 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     plan.blocks_needed = blocks_needed;
     plan.grid = grid;
     plan.lanes = lanes;
+    plan.rec_grid = rec_grid;
+    plan.wide = wide != 0;
     plan.steps_need = steps_need;
     plan.WS = WS;
     plan.W = W;
@@ -1489,22 +1523,32 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
         if (eager) { HIP_CHECK(c, hipEventRecord(c->ev[1], c->stream)); }
         const Args args{ c->m, c->pool, lists, t, fate, c->d_seed, c->d_counters, (int32_t)k0, (int32_t)k1, plan.lanes,
             plan.lanes < WAVE ? 1u : QUEUE_CLAIM };
-        launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, args);
+        if (rec && plan.wide) {
+            const dim3 wg((unsigned)plan.rec_grid), wb(WIDE_BLOCK);
+            if (c->multi_stream) {
+                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, true, WIDE_BLOCK, double>), wg, wb, lds, c->stream, args);
+            } else {
+                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, false, WIDE_BLOCK, double>), wg, wb, lds, c->stream, args);
+            }
+        } else {
+            launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, args);
+        }
         HIP_CHECK(c, hipGetLastError());
         if (eager) { HIP_CHECK(c, hipEventRecord(c->ev[2], c->stream)); }
         if (rec && !global_tally) {
             const int rblocks = (int)((WS + BLOCK - 1) / BLOCK);
             // split the block partials so that the reduce has ~4 blocks per CU
-            const int splits = std::max(1, std::min(grid, (4 * c->n_cu + rblocks - 1) / rblocks));
-            const int per = (grid + splits - 1) / splits;
-            const dim3 rg(rblocks, (unsigned)((grid + per - 1) / per));
+            const int parts = plan.rec_grid;
+            const int splits = std::max(1, std::min(parts, (4 * c->n_cu + rblocks - 1) / rblocks));
+            const int per = (parts + splits - 1) / splits;
+            const dim3 rg(rblocks, (unsigned)((parts + per - 1) / per));
             if (c->tally_fp32) {
                 hipLaunchKernelGGL(reduce_kernel<float>, rg, dim3(BLOCK), 0, c->stream, c->d_pcnt,
                     reinterpret_cast<const float*>(c->d_pfx), reinterpret_cast<const float*>(c->d_pfy), c->d_pcx, c->d_pcy,
-                    grid, per, (int)WS, S, k0, P.step_adjustment, R, c->d_counts, c->d_flux);
+                    parts, per, (int)WS, S, k0, P.step_adjustment, R, c->d_counts, c->d_flux);
             } else {
                 hipLaunchKernelGGL(reduce_kernel<double>, rg, dim3(BLOCK), 0, c->stream, c->d_pcnt, c->d_pfx, c->d_pfy,
-                    c->d_pcx, c->d_pcy, grid, per, (int)WS, S, k0, P.step_adjustment, R, c->d_counts, c->d_flux);
+                    c->d_pcx, c->d_pcy, parts, per, (int)WS, S, k0, P.step_adjustment, R, c->d_counts, c->d_flux);
             }
             HIP_CHECK(c, hipGetLastError());
         }
@@ -1855,6 +1899,10 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     if (!c->d_counts || !c->d_flux || !c->d_dcnt || !c->d_dfx || !c->d_dfy) {
         free_tallies(c);
         return fail(c, PSIM_E_DEVICE, "hipMalloc failed for tallies");
+    }
+    c->flight_cap = sensors[0].flight_cap;
+    for (const Sensor& q : sensors) {
+        if (q.flight_cap != c->flight_cap) { c->flight_cap = 0; }
     }
     c->n_sensors = g->n_sensors;
     c->n_cells = g->n_cells;
