@@ -1087,13 +1087,15 @@ __global__ void bias_grad_kernel(const uint16_t* __restrict__ dz_t, float* __res
 // copies: [in][out] at w_off in pb, [out][in] at w_off in pbT, and for networks of the fused kernels
 // (fused_hidden) in fragment order at f_off in pbF: the 64 lanes' 16-byte operands of one
 // 16 x 16 x 32 product (column n % 16 and K columns 8 (lane / 16) .. of chunk k / 32) lie one after
-// the other, column tiles n / 16 outermost, so a wave reads a fragment as one kilobyte.
+// the other, column tiles n / 16 outermost, so a wave reads a fragment as one kilobyte.  The backward
+// pass reads the hidden matrices transposed, in the same order at r_off.
 constexpr int MAX_WEIGHTS = 17;
 struct LayerTable {
     int count;
     int64_t w_off[MAX_WEIGHTS];
     int in[MAX_WEIGHTS], out[MAX_WEIGHTS];
     int64_t f_off[MAX_WEIGHTS];
+    int64_t r_off[MAX_WEIGHTS];  // the same of the transposed matrix, hidden x hidden ones only (else -1)
 };
 
 __host__ __device__ inline int64_t fragment_index(int k, int n, int in) {
@@ -1110,6 +1112,7 @@ __device__ inline void store_bf16_copies(const LayerTable& lt, int64_t i, uint16
             const uint32_t k = (uint32_t)o / (uint32_t)lt.out[l], n = (uint32_t)o % (uint32_t)lt.out[l];
             pbT[lt.w_off[l] + (int64_t)n * lt.in[l] + k] = b;
             if (pbF) { pbF[lt.f_off[l] + fragment_index((int)k, (int)n, lt.in[l])] = b; }
+            if (pbF && lt.r_off[l] >= 0) { pbF[lt.r_off[l] + fragment_index((int)n, (int)k, lt.out[l])] = b; }
             return;
         }
     }
@@ -1134,11 +1137,18 @@ __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, 
     store_bf16_copies(lt, i, f32_to_bf16(v), pb, pbT, pbF);
 }
 
-// bf16 copies of the FP32 parameters.
-__global__ void params_bf16_kernel(const float* __restrict__ p, uint16_t* __restrict__ pb, uint16_t* __restrict__ pbT,
+// New FP32 parameters: those of the padded output columns are set to zero, the optimiser's state too,
+// and the bf16 copies written.
+__global__ void params_bf16_kernel(float* __restrict__ p, const float* __restrict__ mask, float* __restrict__ m1,
+    float* __restrict__ m2, uint16_t* __restrict__ pb, uint16_t* __restrict__ pbT,
     uint16_t* __restrict__ pbF, LayerTable lt, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
-    if (i < n) { store_bf16_copies(lt, i, f32_to_bf16(p[i]), pb, pbT, pbF); }
+    if (i >= n) { return; }
+    const float v = mask[i] != 0.f ? p[i] : 0.f;
+    p[i] = v;
+    m1[i] = 0.f;
+    m2[i] = 0.f;
+    store_bf16_copies(lt, i, f32_to_bf16(v), pb, pbT, pbF);
 }
 
 __global__ void to_bf16_kernel(const float* __restrict__ x, uint16_t* __restrict__ y, int64_t n) {
@@ -1288,6 +1298,416 @@ __global__ void __launch_bounds__(64 * WAVES) mlp_forward_kernel(MlpArgs p) {
     if (kq == 0 && r < p.rows) { p.y[r] = out[0] + p.p[p.b_off[p.layers]]; }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Training of such a network in three kernels: mlp_train_kernel takes 16 TM rows through the forward
+// pass, the loss and the chain of input gradients; mlp_grad_kernel computes every layer's weight and
+// bias gradients; adam_fused_kernel adds the weight gradients' partial products and steps.  Layer by
+// layer a step was 25 launches of 5-12 us whose operands went out to memory and back twice.  A step of
+// 4096 rows 124 us (56 + 22 + 13 in the kernels), was 261 (220); gradients of 5003 rows 0.35 ms, was
+// 0.99 (their rows, not a multiple of eight, made the weight gradients load element by element).
+// Between the first two, activations and gradients are kept in fragment order over the rows
+// (row_fragment): the operands of the weight gradients' products, whose K is the batch.
+__host__ __device__ inline int64_t row_fragment(int feature, int row, int chunks) {
+    return ((int64_t)(feature / 16) * chunks + row / 32) * 512 + ((row % 32) / 8 * 16 + feature % 16) * 8 + row % 8;
+}
+
+struct TrainArgs {
+    MlpArgs f;  // inputs, weights
+    const float* t;  // [rows] targets
+    uint16_t* a;  // every layer's input in row fragments, at a_off
+    uint16_t* d;  // every layer's output gradient in row fragments, at d_off
+    float* loss;  // [rows] (y - t)^2 / rows
+    const float* consts_from;  // the optimiser's constants of the step (pinned), copied to consts (null: none)
+    float* consts;
+    int chunks;  // 32-row chunks of the batch
+    int64_t r_off[MAX_WEIGHTS], a_off[MAX_WEIGHTS], d_off[MAX_WEIGHTS];
+};
+
+// One block's rows.  Every layer's activations stay in LDS: they are the next layer's operand, and on
+// the way back the ReLU's mask, over which the gradient is written (the lane that reads a mask
+// writes the gradient of the same elements).  Rows past the batch's end carry zeros.
+template <int TM, int TN, int WAVES, int AHEAD>
+__global__ void __launch_bounds__(64 * WAVES) mlp_train_kernel(TrainArgs q) {
+    constexpr int HID = 16 * TN * WAVES, ROWS = 16 * TM, SLOTS = HID / 8, NC = HID / 32;
+    static_assert(NC % AHEAD == 0 && TM <= WAVES, "chunks go round the ring; one wave per row group at the loss");
+    extern __shared__ __attribute__((aligned(16))) unsigned char mlp_smem[];
+    __shared__ float d_out[ROWS];
+    const MlpArgs& p = q.f;
+    auto base = reinterpret_cast<u32x4 (*)[SLOTS]>(mlp_smem);
+    const auto slot = [&](int l) { return base + (int64_t)(l - 1) * ROWS; };  // hidden layer l = 1 .. layers
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, col = lane % 16, kq = lane / 16;
+    const int row0 = blockIdx.x * ROWS, L = p.layers;
+    if (blockIdx.x == 0 && q.consts_from && threadIdx.x < 3) { q.consts[threadIdx.x] = q.consts_from[threadIdx.x]; }
+
+    u32x4 ring[AHEAD][TN];
+    const auto issue = [&](int64_t off, int c, u32x4* r) {
+        const uint16_t* f = p.w + off + ((int64_t)(wave * TN) * NC + c) * 512 + lane * 8;
+        #pragma unroll
+        for (int j = 0; j < TN; ++j) { r[j] = *reinterpret_cast<const u32x4*>(f + (int64_t)j * NC * 512); }
+    };
+    const auto fill = [&](int64_t off) {
+        #pragma unroll
+        for (int u = 0; u < AHEAD; ++u) { issue(off, u, ring[u]); }
+    };
+    if (L > 1) { fill(p.f_off[1]); }
+    // inputs into the last layer's slot (written last), and in row fragments
+    auto X0 = slot(L);
+    load_inputs<ROWS, SLOTS, 64 * WAVES>(p, row0, X0);
+    __syncthreads();
+    for (int v = threadIdx.x; v < p.n_in * (ROWS / 8); v += 64 * WAVES) {  // eight rows of a feature
+        const int feature = v / (ROWS / 8), r = v % (ROWS / 8) * 8;
+        uint32_t w[4];
+        #pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint16_t b = reinterpret_cast<const uint16_t*>(&X0[r + e][(feature / 8) ^ ((r + e) & 15)])[feature % 8];
+            w[e / 2] = e % 2 ? w[e / 2] | (uint32_t)b << 16 : b;
+        }
+        *reinterpret_cast<u32x4*>(q.a + q.a_off[0] + row_fragment(feature, row0 + r, q.chunks)) = u32x4{ w[0], w[1], w[2], w[3] };
+    }
+
+    f32x4 acc[TM][TN];
+    const auto clear = [&]() {
+        #pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            #pragma unroll
+            for (int j = 0; j < TN; ++j) { acc[i][j] = f32x4{ 0.f, 0.f, 0.f, 0.f }; }
+        }
+    };
+    const auto chunk = [&](u32x4 (*X)[SLOTS], int c, const u32x4* fb) {
+        #pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const bf16x8 fa = __builtin_bit_cast(bf16x8, X[i * 16 + col][(c * 4 + kq) ^ col]);
+            #pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fb[j]), fa, acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    // the lane's four consecutive columns n of row i * 16 + col, in its tile's slot
+    const auto piece = [&](u32x4 (*X)[SLOTS], int i, int n) {
+        return reinterpret_cast<u32x2*>(&X[i * 16 + col][(n / 8) ^ col]) + (n / 4) % 2;
+    };
+    // the same values out in row fragments: after the quad transpose the lane holds column
+    // n + lane % 4 of four consecutive rows
+    const auto put_rows = [&](uint16_t* __restrict__ out, int i, int n, u32x2 w) {
+        if (row0 + i * 16 + col >= p.rows) { w = u32x2{ 0u, 0u }; }
+        const u32x2 t = quad_transpose16(w, lane);
+        *reinterpret_cast<u32x2*>(out + row_fragment(n + (lane & 3), row0 + i * 16 + (col & ~3), q.chunks)) = t;
+    };
+    const auto sweep = [&](u32x4 (*X)[SLOTS], int64_t off, int64_t next_off) {  // a hidden x hidden product
+        clear();
+        for (int c0 = 0; c0 < NC; c0 += AHEAD) {
+            const bool more = c0 + AHEAD < NC;
+            #pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                chunk(X, c0 + u, ring[u]);
+                issue(more ? off : next_off, more ? c0 + AHEAD + u : u, ring[u]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    const auto activate = [&](int l) {  // output of weight matrix l: hidden layer l + 1
+        __syncthreads();  // (the input's slot is the last layer's)
+        auto X = slot(l + 1);
+        #pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = (wave * TN + j) * 16 + 4 * kq;
+            const f32x4 bias = *reinterpret_cast<const f32x4*>(p.p + p.b_off[l] + n);
+            #pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                f32x4 v = acc[i][j] + bias;
+                #pragma unroll
+                for (int e = 0; e < 4; ++e) { v[e] = fmaxf(v[e], 0.f); }
+                const u32x2 w = { pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]) };
+                *piece(X, i, n) = w;
+                put_rows(q.a + q.a_off[l + 1], i, n, w);
+            }
+        }
+        __syncthreads();
+    };
+
+    clear();
+    {
+        const int nc = (p.n_in + 31) / 32;
+        const uint16_t* f = p.w + p.f_off[0] + (int64_t)(wave * TN) * nc * 512 + lane * 8;
+        for (int c = 0; c < nc; ++c) {
+            u32x4 fb[TN];
+            #pragma unroll
+            for (int j = 0; j < TN; ++j) { fb[j] = *reinterpret_cast<const u32x4*>(f + ((int64_t)j * nc + c) * 512); }
+            chunk(X0, c, fb);
+        }
+    }
+    activate(0);
+    // after the last forward matrix the ring starts on the way back, which begins with matrix L - 1
+    for (int l = 1; l < L; ++l) {
+        sweep(slot(l), p.f_off[l], l + 1 < L ? p.f_off[l + 1] : q.r_off[L - 1]);
+        activate(l);
+    }
+    // Output layer and loss: dz[r] = 2 (y - t) / rows in column 0, zeros in the others.
+    if (wave < TM) {
+        f32x4 out = f32x4{ 0.f, 0.f, 0.f, 0.f };
+        const uint16_t* f = p.w + p.f_off[L] + lane * 8;
+        auto X = slot(L);
+        #pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const bf16x8 fa = __builtin_bit_cast(bf16x8, X[wave * 16 + col][(c * 4 + kq) ^ col]);
+            out = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(f + c * 512)),
+                fa, out, 0, 0, 0);
+        }
+        if (kq == 0) {
+            const int r = row0 + wave * 16 + col;
+            float v = 0.f;
+            if (r < p.rows) {
+                const float d = out[0] + p.p[p.b_off[L]] - q.t[r];
+                q.loss[r] = d * d / (float)p.rows;
+                v = 2.f * d / (float)p.rows;
+            }
+            d_out[wave * 16 + col] = bf16_to_f32(f32_to_bf16(v));
+        }
+    }
+    __syncthreads();
+    for (int v = threadIdx.x; v < 16 * (ROWS / 8); v += 64 * WAVES) {  // eight rows of an output column
+        const int feature = v / (ROWS / 8), r = v % (ROWS / 8) * 8;
+        u32x4 w = u32x4{ 0u, 0u, 0u, 0u };
+        if (feature == 0) {
+            #pragma unroll
+            for (int e = 0; e < 4; ++e) { w[e] = pack_bf16x2(d_out[r + 2 * e], d_out[r + 2 * e + 1]); }
+        }
+        *reinterpret_cast<u32x4*>(q.d + q.d_off[L] + row_fragment(feature, row0 + r, q.chunks)) = w;
+    }
+    // Gradient v of hidden layer l through its ReLU: in place of the activation, and in row fragments.
+    const auto mask_out = [&](int l, int i, int n, f32x4 v) {
+        u32x2* at = piece(slot(l), i, n);
+        const u32x2 mk = *at;
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool on = bf16_to_f32((uint16_t)(mk[e / 2] >> (16 * (e % 2)))) > 0.f;
+            v[e] = on && row0 + i * 16 + col < p.rows ? v[e] : 0.f;
+        }
+        const u32x2 w = { pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]) };
+        *at = w;
+        put_rows(q.d + q.d_off[l - 1], i, n, w);
+    };
+    #pragma unroll
+    for (int j = 0; j < TN; ++j) {  // the output layer's product has one column: exact in FP32
+        const int n = (wave * TN + j) * 16 + 4 * kq;
+        const u32x2 w = *reinterpret_cast<const u32x2*>(p.w + p.f_off[L] + fragment_index(n, 0, HID));
+        #pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const float d = d_out[i * 16 + col];
+            f32x4 v;
+            #pragma unroll
+            for (int e = 0; e < 4; ++e) { v[e] = d * bf16_to_f32((uint16_t)(w[e / 2] >> (16 * (e % 2)))) + 0.f; }
+            mask_out(L, i, n, v);
+        }
+    }
+    __syncthreads();
+    for (int l = L - 1; l > 0; --l) {
+        sweep(slot(l + 1), q.r_off[l], l > 1 ? q.r_off[l - 1] : q.r_off[l]);
+        #pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            #pragma unroll
+            for (int i = 0; i < TM; ++i) { mask_out(l, i, (wave * TN + j) * 16 + 4 * kq, acc[i][j]); }
+        }
+        __syncthreads();
+    }
+}
+
+// Weight gradients dW = a^T dz of all layers, then the bias gradients.  A block of 8 waves computes a
+// 128 x 256 tile of one layer over one split of the rows, each wave 64 x 64, both operands straight
+// from their row fragments (a kilobyte per load; waves of a block share them in L1); no LDS, no
+// barrier.  Splits, and the order of every sum, are those of the products (nt_splits).  The partial
+// products go to ws and are added in split order by whoever reads them.
+constexpr int GRAD_BM = 128, GRAD_BN = 256, GRAD_AHEAD = 2;  // chunks in flight (3 and 4: 5-8% slower)
+
+struct GradArgs {
+    const uint16_t* a;
+    const uint16_t* d;
+    float* ws;
+    float* g;  // flat gradient (bias entries written here)
+    int count, chunks, rows;
+    int bias_first;  // first block of the bias gradients
+    int64_t a_off[MAX_WEIGHTS], d_off[MAX_WEIGHTS], ws_off[MAX_WEIGHTS], b_off[MAX_WEIGHTS];
+    int in[MAX_WEIGHTS], out[MAX_WEIGHTS], splits[MAX_WEIGHTS], split_chunks[MAX_WEIGHTS], first[MAX_WEIGHTS], bias_tile[MAX_WEIGHTS];
+};
+
+__global__ void __launch_bounds__(512) mlp_grad_kernel(GradArgs q) {
+    __shared__ float part[16][257];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, col = lane % 16, kq = lane / 16;
+    int b = blockIdx.x, l = q.count - 1;
+    if (b >= q.bias_first) {
+        // db[c] = the column's sum over the rows, as bias_grad_kernel adds it: 256 partial sums of every
+        // 256th row, then a tree.  Wave w holds rows 32 w .. 32 w + 31 of each 256.
+        b -= q.bias_first;
+        while (b < q.bias_tile[l]) { --l; }
+        const int tile = b - q.bias_tile[l];
+        float s[8] = { 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f };
+        const uint16_t* f = q.d + q.d_off[l] + (int64_t)tile * q.chunks * 512 + lane * 8;
+        for (int c = wave; c < q.chunks; c += 8) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(f + (int64_t)c * 512);
+            #pragma unroll
+            for (int e = 0; e < 8; ++e) { s[e] += bf16_to_f32((uint16_t)(v[e / 2] >> (16 * (e % 2)))); }
+        }
+        #pragma unroll
+        for (int e = 0; e < 8; ++e) { part[col][wave * 32 + kq * 8 + e] = s[e]; }
+        __syncthreads();
+        for (int off = 128; off > 0; off >>= 1) {
+            for (int k = threadIdx.x; k < 16 * off; k += 512) { part[k / off][k % off] += part[k / off][k % off + off]; }
+            __syncthreads();
+        }
+        if (threadIdx.x < 16) { q.g[q.b_off[l] + tile * 16 + threadIdx.x] = part[threadIdx.x][0]; }
+        return;
+    }
+    while (b < q.first[l]) { --l; }
+    b -= q.first[l];
+    const int in = q.in[l], out = q.out[l], tiles_m = (in + GRAD_BM - 1) / GRAD_BM, tiles_n = (out + GRAD_BN - 1) / GRAD_BN;
+    // Blocks go to the XCDs in turn; each takes a run of neighbouring units, tiles fastest, so that the
+    // tiles of a split, which read the same rows, share an L2 (4096 rows 22 us, dealt out singly 31).
+    const int units = q.splits[l] * tiles_m * tiles_n;
+    if (units % XCDS == 0) { b = b % XCDS * (units / XCDS) + b / XCDS; }
+    const int split = b / (tiles_m * tiles_n), tile = b % (tiles_m * tiles_n);
+    const int m0 = tile / tiles_n * GRAD_BM + wave / 4 * 64, n0 = tile % tiles_n * GRAD_BN + wave % 4 * 64;
+    const int tm = min(4, (in - m0 + 15) / 16), tn = min(4, (out - n0 + 15) / 16);  // 16-wide tiles this wave has
+    if (tm <= 0 || tn <= 0) { return; }
+    const int c0 = split * q.split_chunks[l], c1 = min(q.chunks, c0 + q.split_chunks[l]);
+    const uint16_t* fa = q.a + q.a_off[l] + (int64_t)(m0 / 16) * q.chunks * 512 + lane * 8;
+    const uint16_t* fb = q.d + q.d_off[l] + (int64_t)(n0 / 16) * q.chunks * 512 + lane * 8;
+    const int64_t pitch = (int64_t)q.chunks * 512;
+    u32x4 ra[GRAD_AHEAD][4], rb[GRAD_AHEAD][4];
+    const auto issue = [&](int c, u32x4* a, u32x4* d) {
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {  // a tile that is not there repeats the wave's last (its sums are not stored)
+            a[i] = *reinterpret_cast<const u32x4*>(fa + min(i, tm - 1) * pitch + (int64_t)c * 512);
+            d[i] = *reinterpret_cast<const u32x4*>(fb + min(i, tn - 1) * pitch + (int64_t)c * 512);
+        }
+    };
+    f32x4 acc[4][4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) { acc[i][j] = f32x4{ 0.f, 0.f, 0.f, 0.f }; }
+    }
+    #pragma unroll
+    for (int u = 0; u < GRAD_AHEAD; ++u) { issue(min(c0 + u, c1 - 1), ra[u], rb[u]); }
+    for (int c = c0; c < c1; c += GRAD_AHEAD) {
+        #pragma unroll
+        for (int u = 0; u < GRAD_AHEAD; ++u) {
+            if (c + u < c1) {
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    #pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, rb[u][j]),
+                            __builtin_bit_cast(bf16x8, ra[u][i]), acc[i][j], 0, 0, 0);
+                    }
+                }
+            }
+            issue(min(c + u + GRAD_AHEAD, c1 - 1), ra[u], rb[u]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    float* __restrict__ C = q.ws + q.ws_off[l] + (int64_t)split * in * out;
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + i * 16 + col;
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (i < tm && j < tn && m < in) { *reinterpret_cast<f32x4*>(C + (int64_t)m * out + n0 + j * 16 + 4 * kq) = acc[i][j]; }
+        }
+    }
+}
+
+// Where the partial weight gradients lie and how many there are of each layer.
+struct PartTable {
+    LayerTable lt;
+    int64_t b_off[MAX_WEIGHTS], ws_off[MAX_WEIGHTS];
+    int splits[MAX_WEIGHTS];
+    int64_t first[MAX_WEIGHTS];  // first item of a layer: one per ADAM_ROWS rows x 1 column of its matrix, then its biases
+};
+
+// Flat gradient from the partial products (the biases are there already).
+__global__ void sum_parts_kernel(const float* __restrict__ ws, float* __restrict__ g, PartTable q, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (i >= n) { return; }
+    for (int l = 0; l < q.lt.count; ++l) {
+        const int64_t size = (int64_t)q.lt.in[l] * q.lt.out[l], o = i - q.lt.w_off[l];
+        if (o >= 0 && o < size) {
+            float s = 0.f;
+            for (int z = 0; z < q.splits[l]; ++z) { s += ws[q.ws_off[l] + z * size + o]; }
+            g[i] = s;
+            return;
+        }
+    }
+}
+
+__device__ inline float adam_step(float& p, float g, float& m1, float& m2, float lr, float c1, float c2, float b1, float b2,
+    float eps) {
+    const float a = b1 * m1 + (1.f - b1) * g;
+    const float b = b2 * m2 + (1.f - b2) * g * g;
+    m1 = a;
+    m2 = b;
+    p = p - lr * (a / c1) / (sqrtf(b / c2) + eps);
+    return p;
+}
+
+// adam_kernel with the weight gradients' partial products added on the way in.  A thread takes four
+// consecutive rows of one column: loads and [in][out] stores of a wave stay contiguous, and the
+// copies that run along a column ([out][in] and fragment order) are 8-byte stores.
+constexpr int ADAM_ROWS = 4;
+
+__global__ void __launch_bounds__(EW_BLOCK) adam_fused_kernel(float* __restrict__ p, const float* __restrict__ ws,
+    const float* __restrict__ g, float* __restrict__ m1, float* __restrict__ m2, const float* __restrict__ mask,
+    uint16_t* __restrict__ pb, uint16_t* __restrict__ pbT, uint16_t* __restrict__ pbF, PartTable q, int64_t items,
+    const float* __restrict__ step_consts, float b1, float b2, float eps) {
+    const int64_t item = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (item >= items) { return; }
+    const float lr = step_consts[0], c1 = step_consts[1], c2 = step_consts[2];
+    int l = q.lt.count - 1;
+    while (item < q.first[l]) { --l; }
+    const int in = q.lt.in[l], out = q.lt.out[l];
+    const uint32_t o = (uint32_t)(item - q.first[l]), groups = (uint32_t)((in + ADAM_ROWS - 1) / ADAM_ROWS);
+    if (o >= groups * (uint32_t)out) {  // a bias
+        const int64_t i = q.b_off[l] + (o - groups * (uint32_t)out);
+        pb[i] = f32_to_bf16(adam_step(p[i], g[i] * mask[i], m1[i], m2[i], lr, c1, c2, b1, b2, eps));
+        return;
+    }
+    const int n = (int)(o % (uint32_t)out), k0 = (int)(o / (uint32_t)out) * ADAM_ROWS;
+    const int64_t size = (int64_t)in * out, w0 = q.lt.w_off[l];
+    const int rows = min(ADAM_ROWS, in - k0);
+    float s[ADAM_ROWS];
+    #pragma unroll
+    for (int j = 0; j < ADAM_ROWS; ++j) { s[j] = 0.f; }
+    const float* __restrict__ part = ws + q.ws_off[l] + (int64_t)k0 * out + n;
+    #pragma unroll 8
+    for (int z = 0; z < q.splits[l]; ++z, part += size) {
+        #pragma unroll
+        for (int j = 0; j < ADAM_ROWS; ++j) { s[j] += part[(int64_t)min(j, rows - 1) * out]; }
+    }
+    uint16_t v[ADAM_ROWS];
+    #pragma unroll
+    for (int j = 0; j < ADAM_ROWS; ++j) {
+        v[j] = 0;
+        if (j < rows) {
+            const int64_t i = w0 + (int64_t)(k0 + j) * out + n;
+            v[j] = f32_to_bf16(adam_step(p[i], s[j] * mask[i], m1[i], m2[i], lr, c1, c2, b1, b2, eps));
+            pb[i] = v[j];
+            if (q.lt.r_off[l] >= 0) { pbF[q.lt.r_off[l] + fragment_index(n, k0 + j, out)] = v[j]; }
+        }
+    }
+    u32x2 w;
+    std::memcpy(&w, v, 8);
+    *reinterpret_cast<u32x2*>(pbF + q.lt.f_off[l] + fragment_index(k0, n, in)) = w;  // rows past `in` are its padding
+    uint16_t* col = pbT + w0 + (int64_t)n * in + k0;
+    if (in % ADAM_ROWS == 0) {
+        *reinterpret_cast<u32x2*>(col) = w;
+    } else {
+        #pragma unroll
+        for (int j = 0; j < ADAM_ROWS; ++j) {
+            if (j < rows) { col[j] = v[j]; }
+        }
+    }
+}
+
 constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(64) << 20;
 
 }  // namespace
@@ -1310,7 +1730,7 @@ struct psim_mlp {
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr, *mask = nullptr;
     uint16_t* pb = nullptr;  // bf16 copy, layout of p (weights [in][out]; biases unused)
     uint16_t* pbF = nullptr;  // bf16 weights in fragment order (fused kernels; null: not such a network)
-    std::vector<int64_t> f_off;  // their offsets
+    std::vector<int64_t> f_off, r_off;  // their offsets, as the products' operand and transposed (LayerTable)
     uint16_t* pbT = nullptr;  // bf16 weights transposed, [out][in] per layer (K-major for the forward)
     float* ws = nullptr;  // partial products of weight gradients split over K
     size_t ws_elems = 0;
@@ -1334,6 +1754,13 @@ struct psim_mlp {
     std::vector<uint16_t*> aT;  // aT[l]: a[l] transposed
     uint16_t *dz = nullptr, *dz2 = nullptr;  // bf16 gradient of the current layer's pre-activation [rows][features]
     uint16_t *dzT = nullptr, *dz2T = nullptr;  // the same transposed
+    // the fused training kernels: activations and gradients in row fragments (frag_rows rows of them),
+    // partial weight gradients of all layers (parts_elems)
+    uint16_t *frag_a = nullptr, *frag_d = nullptr;
+    int frag_rows = 0;
+    float* parts = nullptr;
+    int64_t parts_elems = 0;
+    float* h_loss = nullptr;  // pinned: targets (moderate calls) and loss terms, frag_rows of each
     // device address of this GPU's `scratch` array (psim_mlp_forward_noalloc), looked up at create
     unsigned char* scratch = nullptr;
     // training steps replayed from a HIP graph: the step's kernels (forward, backward, Adam) captured
@@ -1345,6 +1772,7 @@ struct psim_mlp {
     hipGraphExec_t graph_exec = nullptr;
     int graph_rows = 0;  // batch size of the captured step (0: none)
     int64_t graph_gen = 0;  // alloc_gen when it was captured
+    bool graph_fused = false;  // captured on the fused kernels
     int warm_rows = 0;  // batch size of the last eager step
     int64_t alloc_gen = 0;  // bumped when batch or training buffers move
 };
@@ -1475,6 +1903,7 @@ LayerTable layer_table(const psim_mlp* h) {
         lt.in[l] = h->dims[l];
         lt.out[l] = h->dims[l + 1];
         lt.f_off[l] = h->f_off.empty() ? 0 : h->f_off[l];
+        lt.r_off[l] = h->r_off.empty() ? -1 : h->r_off[l];
     }
     return lt;
 }
@@ -1685,6 +2114,179 @@ int read_loss(psim_mlp* h, int rows, float* loss) {
     return PSIM_OK;
 }
 
+// ---- the fused training step ----------------------------------------------------------------
+
+constexpr int LDS_BYTES = 160 * 1024 - 1024;  // per CU, less the kernels' static arrays
+
+// Row groups of 16 per block of mlp_train_kernel: two where every layer's activations of 32 rows fit
+// LDS (32 -> 512 x 4: 4096 rows 55.9 us against 59.2 with one, 8192 69.2 against 106.5, 64 the same).
+int train_groups(const psim_mlp* h) { return std::min(2, LDS_BYTES / (16 * h->hidden * 2 * h->layers)); }
+
+bool fused_train(const psim_mlp* h) { return fused_forward(h) && train_groups(h) >= 1; }
+
+void free_frags(psim_mlp* h) {
+    for (uint16_t* q : { h->frag_a, h->frag_d }) {
+        if (q) { (void)hipFree(q); }
+    }
+    if (h->h_loss) { (void)hipHostFree(h->h_loss); }
+    h->frag_a = h->frag_d = nullptr;
+    h->h_loss = nullptr;
+    h->frag_rows = 0;
+}
+
+int pad16(int n) { return (n + 15) / 16 * 16; }
+
+// Splits of layer l's weight gradient over `rows`, and the 32-row chunks of each: launch_nt's.
+int part_splits(const psim_mlp* h, int l, int rows, int* chunks) {
+    int splits = nt_splits(h->dims[l], h->dims[l + 1], rows);
+    int k_split = (rows + KB - 1) / KB * KB;
+    if (splits > 1) {
+        k_split = ((rows + splits - 1) / splits + KB - 1) / KB * KB;
+        splits = (rows + k_split - 1) / k_split;
+    }
+    *chunks = k_split / 32;
+    return splits;
+}
+
+int ensure_frags(psim_mlp* h, int rows) {
+    int64_t parts = 0;
+    for (int l = 0; l <= h->layers; ++l) {
+        int chunks = 0;
+        parts += (int64_t)part_splits(h, l, rows, &chunks) * h->dims[l] * h->dims[l + 1];
+    }
+    if (parts > h->parts_elems) {
+        if (h->parts) { (void)hipFree(h->parts); }
+        h->parts = mlp_alloc<float>((size_t)parts);
+        h->parts_elems = h->parts ? parts : 0;
+        h->alloc_gen++;
+        if (!h->parts) { return mlp_fail(h, PSIM_E_DEVICE, "hipMalloc failed for the surrogate partial gradients"); }
+    }
+    if (rows <= h->frag_rows) { return PSIM_OK; }
+    free_frags(h);
+    const int cap = (rows + 63) / 64 * 64;
+    size_t fa = 0, fd = 0;
+    for (int l = 0; l <= h->layers; ++l) {
+        fa += (size_t)pad16(h->dims[l]);
+        fd += (size_t)h->dims[l + 1];
+    }
+    h->frag_a = mlp_alloc<uint16_t>(fa * (size_t)cap);
+    h->frag_d = mlp_alloc<uint16_t>(fd * (size_t)cap);
+    if (hipHostMalloc(reinterpret_cast<void**>(&h->h_loss), 2 * sizeof(float) * (size_t)cap, hipHostMallocDefault) != hipSuccess) {
+        h->h_loss = nullptr;
+    }
+    if (!h->frag_a || !h->frag_d || !h->h_loss) {
+        free_frags(h);
+        return mlp_fail(h, PSIM_E_DEVICE, "hipMalloc failed for the surrogate training buffers");
+    }
+    h->frag_rows = cap;
+    h->alloc_gen++;
+    return PSIM_OK;
+}
+
+template <int TM, int TN>
+void launch_mlp_train(const TrainArgs& a, hipStream_t st) {
+    constexpr int WAVES = 8;
+    const int blocks = a.chunks * 2 / TM;  // whole chunks, whose rows past the end are written as zeros
+    const size_t lds = (size_t)16 * TM * 16 * TN * WAVES * 2 * a.f.layers;
+    hipLaunchKernelGGL((mlp_train_kernel<TM, TN, WAVES, (TM == 1 ? 8 : 4)>), dim3((unsigned)blocks), dim3(64 * WAVES), lds, st, a);
+}
+
+// Inputs where the fused kernels read them: pinned memory for calls of moderate size, else copies on
+// the device.
+int load_fused(psim_mlp* h, const float* x, const float* t, int rows, const float** dx, const float** dt) {
+    int rc;
+    if ((rc = ensure_frags(h, rows)) != 0) { return rc; }
+    const size_t in_bytes = sizeof(float) * (size_t)rows * h->n_in;
+    std::memcpy(h->h_loss + h->frag_rows, t, sizeof(float) * (size_t)rows);
+    *dt = h->h_loss + h->frag_rows;
+    if (in_bytes <= PINNED_BYTES) {
+        std::memcpy(h->h_x, x, in_bytes);
+        *dx = h->h_x;
+        return PSIM_OK;
+    }
+    if ((rc = ensure_io(h, rows)) != 0) { return rc; }
+    MLP_CHECK(h, hipMemcpyAsync(h->xin, x, in_bytes, hipMemcpyHostToDevice, h->stream));
+    *dx = h->xin;
+    return PSIM_OK;
+}
+
+// The gradient kernels of one batch; the weight gradients' partial products stay in h->parts, laid out
+// as `parts` says.  `step`: also moves the step's constants to the device.
+int fused_gradients(psim_mlp* h, const float* x, const float* t, int rows, bool step, PartTable* parts, int64_t* items) {
+    TrainArgs a{};
+    GradArgs g{};
+    PartTable& q = *parts;
+    q = PartTable{};
+    q.lt = layer_table(h);
+    a.f.x = x;
+    a.f.w = h->pbF;
+    a.f.p = h->p;
+    a.f.rows = rows;
+    a.f.n_in = h->n_in;
+    a.f.layers = h->layers;
+    a.t = t;
+    a.a = h->frag_a;
+    a.d = h->frag_d;
+    a.loss = h->h_loss;
+    a.consts_from = step ? h->h_step_consts : nullptr;
+    a.consts = h->step_consts;
+    a.chunks = g.chunks = (rows + 31) / 32;
+    g.a = h->frag_a;
+    g.d = h->frag_d;
+    g.ws = h->parts;
+    g.g = h->g;
+    g.rows = rows;
+    g.count = h->layers + 1;
+    int64_t oa = 0, od = 0, ow = 0, oi = 0;
+    int blocks = 0, tiles = 0;
+    for (int l = 0; l <= h->layers; ++l) {
+        const int in = h->dims[l], out = h->dims[l + 1];
+        a.f.f_off[l] = h->f_off[l];
+        a.f.b_off[l] = h->b_off[l];
+        a.r_off[l] = h->r_off[l];
+        a.a_off[l] = g.a_off[l] = oa;
+        a.d_off[l] = g.d_off[l] = od;
+        oa += (int64_t)pad16(in) * a.chunks * 32;
+        od += (int64_t)out * a.chunks * 32;
+        q.splits[l] = g.splits[l] = part_splits(h, l, rows, &g.split_chunks[l]);
+        q.ws_off[l] = g.ws_off[l] = ow;
+        ow += (int64_t)q.splits[l] * in * out;
+        q.b_off[l] = g.b_off[l] = h->b_off[l];
+        g.in[l] = in;
+        g.out[l] = out;
+        g.first[l] = blocks;
+        blocks += q.splits[l] * ((in + GRAD_BM - 1) / GRAD_BM) * ((out + GRAD_BN - 1) / GRAD_BN);
+        g.bias_tile[l] = tiles;
+        tiles += out / 16;
+        q.first[l] = oi;
+        oi += (int64_t)((in + ADAM_ROWS - 1) / ADAM_ROWS) * out + out;
+    }
+    g.bias_first = blocks;
+    *items = oi;
+    if (train_groups(h) == 2) {
+        if (h->hidden == 512) {
+            launch_mlp_train<2, 4>(a, h->stream);
+        } else {
+            launch_mlp_train<2, 2>(a, h->stream);
+        }
+    } else if (h->hidden == 512) {
+        launch_mlp_train<1, 4>(a, h->stream);
+    } else {
+        launch_mlp_train<1, 2>(a, h->stream);
+    }
+    MLP_CHECK(h, hipGetLastError());
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3((unsigned)(blocks + tiles)), dim3(512), 0, h->stream, g);
+    MLP_CHECK(h, hipGetLastError());
+    return PSIM_OK;
+}
+
+// The mean squared error from the pinned loss terms (in row order), after the stream has ended.
+float sum_loss(const psim_mlp* h, int rows) {
+    double s = 0.;
+    for (int r = 0; r < rows; ++r) { s += h->h_loss[r]; }
+    return (float)s;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1719,6 +2321,11 @@ int psim_mlp_create(psim_mlp** out, int device, int32_t n_in, int32_t hidden, in
         for (size_t l = 0; l + 1 < h->dims.size(); ++l) {
             h->f_off.push_back(f_elems);
             f_elems += (int64_t)((h->dims[l] + 31) / 32 * 32) * h->dims[l + 1];
+        }
+        for (int l = 0; l <= layers; ++l) {
+            const bool square = l > 0 && l < layers;
+            h->r_off.push_back(square ? f_elems : -1);
+            f_elems += square ? (int64_t)hidden * hidden : 0;
         }
         h->pbF = mlp_alloc<uint16_t>((size_t)f_elems);
     }
@@ -1789,6 +2396,8 @@ void psim_mlp_destroy(psim_mlp* h) {
     free_train(h);
     free_batch(h);
     free_io(h);
+    free_frags(h);
+    if (h->parts) { (void)hipFree(h->parts); }
     void* ps[] = { h->p, h->g, h->m1, h->m2, h->mask, h->pb, h->pbT, h->pbF, h->ws, h->counters, h->step_consts };
     for (void* q : ps) {
         if (q) { (void)hipFree(q); }
@@ -1804,19 +2413,10 @@ int64_t psim_mlp_num_params(const psim_mlp* h) { return h ? h->n_params : 0; }
 int psim_mlp_set_params(psim_mlp* h, const float* params) {
     if (!h || !params) { return PSIM_E_INVALID; }
     MLP_CHECK(h, hipSetDevice(h->device));
-    std::vector<float> p(params, params + h->n_params);
-    // padded output columns are forced to zero
-    const int L = (int)h->dims.size() - 1;
-    for (int k = 0; k < h->dims[L - 1]; ++k) {
-        for (int n = 1; n < PAD_OUT; ++n) { p[(size_t)(h->w_off[L - 1] + (int64_t)k * PAD_OUT + n)] = 0.f; }
-    }
-    for (int n = 1; n < PAD_OUT; ++n) { p[(size_t)(h->b_off[L - 1] + n)] = 0.f; }
-    MLP_CHECK(h, hipMemcpy(h->p, p.data(), sizeof(float) * p.size(), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(params_bf16_kernel, dim3(ew_blocks(h->n_params)), dim3(EW_BLOCK), 0, h->stream, h->p, h->pb,
-        h->pbT, h->pbF, layer_table(h), h->n_params);
+    MLP_CHECK(h, hipMemcpyAsync(h->p, params, sizeof(float) * (size_t)h->n_params, hipMemcpyHostToDevice, h->stream));
+    hipLaunchKernelGGL(params_bf16_kernel, dim3(ew_blocks(h->n_params)), dim3(EW_BLOCK), 0, h->stream, h->p, h->mask, h->m1,
+        h->m2, h->pb, h->pbT, h->pbF, layer_table(h), h->n_params);
     MLP_CHECK(h, hipGetLastError());
-    MLP_CHECK(h, hipMemsetAsync(h->m1, 0, sizeof(float) * (size_t)h->n_params, h->stream));
-    MLP_CHECK(h, hipMemsetAsync(h->m2, 0, sizeof(float) * (size_t)h->n_params, h->stream));
     MLP_CHECK(h, hipStreamSynchronize(h->stream));
     h->step = 0;
     return PSIM_OK;
@@ -1917,6 +2517,22 @@ int psim_mlp_gradients(psim_mlp* h, const float* x, const float* t, int32_t rows
     if (rows > MAX_ROWS) { return mlp_fail(h, PSIM_E_INVALID, "more than 4194240 rows in one call"); }
     MLP_CHECK(h, hipSetDevice(h->device));
     int rc;
+    if (fused_train(h)) {
+        const float *dx = nullptr, *dt = nullptr;
+        PartTable parts;
+        int64_t items = 0;
+        if ((rc = load_fused(h, x, t, rows, &dx, &dt)) != 0) { return rc; }
+        if ((rc = fused_gradients(h, dx, dt, rows, false, &parts, &items)) != 0) { return rc; }
+        if (grad) {
+            hipLaunchKernelGGL(sum_parts_kernel, dim3(ew_blocks(h->n_params)), dim3(EW_BLOCK), 0, h->stream, h->parts, h->g,
+                parts, h->n_params);
+            MLP_CHECK(h, hipGetLastError());
+            MLP_CHECK(h, hipMemcpyAsync(grad, h->g, sizeof(float) * (size_t)h->n_params, hipMemcpyDeviceToHost, h->stream));
+        }
+        MLP_CHECK(h, hipStreamSynchronize(h->stream));
+        if (loss) { *loss = sum_loss(h, rows); }
+        return PSIM_OK;
+    }
     if ((rc = load_batch(h, x, t, rows)) != 0) { return rc; }
     if ((rc = forward(h, rows, true)) != 0) { return rc; }
     if ((rc = backward(h, rows)) != 0) { return rc; }
@@ -1933,16 +2549,29 @@ int psim_mlp_train_step(psim_mlp* h, const float* x, const float* t, int32_t row
     if (rows > MAX_ROWS) { return mlp_fail(h, PSIM_E_INVALID, "more than 4194240 rows in one call"); }
     MLP_CHECK(h, hipSetDevice(h->device));
     int rc;
-    if ((rc = load_batch(h, x, t, rows)) != 0) { return rc; }
+    const bool fused = fused_train(h);
+    const float *dx = nullptr, *dt = nullptr;
+    if ((rc = fused ? load_fused(h, x, t, rows, &dx, &dt) : load_batch(h, x, t, rows)) != 0) { return rc; }
     ++h->step;
     const float b1 = 0.9f, b2 = 0.999f;
     h->h_step_consts[0] = lr;
     h->h_step_consts[1] = 1.f - std::pow(b1, (float)h->step);
     h->h_step_consts[2] = 1.f - std::pow(b2, (float)h->step);
-    MLP_CHECK(h, hipMemcpyAsync(h->step_consts, h->h_step_consts, 3 * sizeof(float), hipMemcpyHostToDevice, h->stream));
+    if (!fused) {
+        MLP_CHECK(h, hipMemcpyAsync(h->step_consts, h->h_step_consts, 3 * sizeof(float), hipMemcpyHostToDevice, h->stream));
+    }
     // The step's kernels: forward, backward, Adam (all on h->stream, no host synchronisation).
     const auto enqueue = [&]() -> int {
         int r;
+        if (fused) {
+            PartTable parts;
+            int64_t items = 0;
+            if ((r = fused_gradients(h, dx, dt, rows, true, &parts, &items)) != 0) { return r; }
+            hipLaunchKernelGGL(adam_fused_kernel, dim3(ew_blocks(items)), dim3(EW_BLOCK), 0, h->stream, h->p, h->parts, h->g,
+                h->m1, h->m2, h->mask, h->pb, h->pbT, h->pbF, parts, items, h->step_consts, b1, b2, 1e-8f);
+            MLP_CHECK(h, hipGetLastError());
+            return PSIM_OK;
+        }
         if ((r = forward(h, rows, true)) != 0) { return r; }
         if ((r = backward(h, rows)) != 0) { return r; }
         hipLaunchKernelGGL(adam_kernel, dim3(ew_blocks(h->n_params)), dim3(EW_BLOCK), 0, h->stream, h->p, h->g, h->m1,
@@ -1950,7 +2579,7 @@ int psim_mlp_train_step(psim_mlp* h, const float* x, const float* t, int32_t row
         MLP_CHECK(h, hipGetLastError());
         return PSIM_OK;
     };
-    if (h->graph_rows && (h->alloc_gen != h->graph_gen || h->graph_rows != rows)) {  // buffers moved or another size
+    if (h->graph_rows && (h->alloc_gen != h->graph_gen || h->graph_rows != rows || h->graph_fused != fused)) {  // buffers moved or another size
         if (h->graph_exec) { (void)hipGraphExecDestroy(h->graph_exec); }
         if (h->graph) { (void)hipGraphDestroy(h->graph); }
         h->graph_exec = nullptr;
@@ -1976,11 +2605,13 @@ int psim_mlp_train_step(psim_mlp* h, const float* x, const float* t, int32_t row
             MLP_CHECK(h, hipGraphInstantiate(&h->graph_exec, h->graph, nullptr, nullptr, 0));
             h->graph_rows = rows;
             h->graph_gen = h->alloc_gen;
+            h->graph_fused = fused;
         }
         MLP_CHECK(h, hipGraphLaunch(h->graph_exec, h->stream));
     }
-    if (loss) { return read_loss(h, rows, loss); }
+    if (loss && !fused) { return read_loss(h, rows, loss); }
     MLP_CHECK(h, hipStreamSynchronize(h->stream));
+    if (loss) { *loss = sum_loss(h, rows); }
     return PSIM_OK;
 }
 
