@@ -42,17 +42,16 @@ constexpr int WAVE = 64;
 constexpr int LDS_TALLY_BYTES = 48 * 1024;  // budget for one block's [W][S] window tally
 constexpr int LDS_WIDE_BYTES = 160 * 1024;  // the same where one block has a CU to itself
 constexpr int GLOBAL_TALLY_STEPS = 16;  // fewer LDS-tallied steps per window than this: HBM tallies
-// Fewer phonons per sensor than this: global atomics too.  Small runs lose more to the many short
-// LDS windows (launches, reductions, sorts) than HBM atomics lose to contention, large ones the
-// reverse (measured at 1e4 and 1e5 phonons per sensor: 1.8-3x faster in HBM below, 2.7x slower
-// above).
-constexpr int64_t LDS_MIN_PHONONS_PER_SENSOR = 30000;
-// The same with wide windows (wide_window_for) of at least WIDE_LDS_STEPS steps, of which a run has few:
-// film of 3e5 phonons (10000 per sensor) 14.2 ms in LDS, 30.4 in HBM; L-shape of 3e5 (7500) periodic
-// 18.1 against 26.3, steady state 17.5 against 17.6; with 69-step windows (bar of 100 sensors) LDS
-// still loses at 10000 per sensor, 42.3 against 34.5.
+// Fewer phonons than this in a run: HBM tallies too.  Every LDS window ends with a tail in which the last
+// phonons finish, a sort and a reduction; a run of HBM tallies has one.  Measured with wide windows
+// (wide_window_for), ms in LDS / in HBM, every step recorded: L-shape of 3e5 phonons 17.0 / 12.0, 6e5
+// 20.4 / 20.9, 1e6 25.7 / 30.8; film of 3e5 13.0 / 14.6, 6e5 15.1 / 22.9; bar of 6e5 19.8 / 16.5, 2e6
+// 27.5 / 36.6; bars of 1-4 sensors and 7e4-2.5e5 phonons 5.8-14.9 / 1.2-6.2.
+constexpr int64_t LDS_MIN_PHONONS = 600000;
+// The same where the windows stay shorter than WIDE_LDS_STEPS steps, so that a run has many: the bar of
+// 100 sensors (69 steps a window) 40.9 / 27.9 at 1e4 phonons per sensor, 49.4 / 46.3 at 2e4.
 constexpr int32_t WIDE_LDS_STEPS = 128;
-constexpr int64_t WIDE_MIN_PHONONS_PER_SENSOR = 7500;
+constexpr int64_t LDS_MIN_PHONONS_PER_SENSOR = 30000;
 constexpr uint32_t QUEUE_CLAIM = 32;  // work-queue items a wave claims per atomic
 // A run of fewer phonons than the chip has lanes is as long as its longest-lived phonon: each event
 // waits for the one before.  An iteration costs a wave every stage that any of its lanes is in, so
@@ -1393,7 +1392,8 @@ bool use_global_tally(const psim_gpu_ctx* c) {
     const int64_t lds_steps = LDS_TALLY_BYTES / (20 * sensors) - 1;
     if (c->tally_mode == PSIM_TALLY_HBM || lds_steps < 1) { return true; }
     if (c->tally_mode == PSIM_TALLY_LDS) { return false; }
-    if (wide_window_for(c) >= WIDE_LDS_STEPS) { return c->params.total_phonons < WIDE_MIN_PHONONS_PER_SENSOR * sensors; }
+    if (c->params.total_phonons < LDS_MIN_PHONONS) { return true; }
+    if (wide_window_for(c) >= WIDE_LDS_STEPS) { return false; }
     return lds_steps < GLOBAL_TALLY_STEPS || c->params.total_phonons < LDS_MIN_PHONONS_PER_SENSOR * sensors;
 }
 
