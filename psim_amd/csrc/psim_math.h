@@ -197,7 +197,16 @@ PSIM_QUAL double psim_cos2pi(double u) {
     const double c = (1.0 - 0.5 * z) + (z * z) * pc;
     const double s = a + (a * z) * ps;
     const int qi = (int)q & 3;
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* selected by bits: both series are wanted in a wave, and side by side they fill each other's
+     * latency where branches would run one after the other */
+    const unsigned long long take_s = 0ull - (unsigned long long)(qi & 1);
+    const unsigned long long bits = (__builtin_bit_cast(unsigned long long, s) & take_s)
+                                    | (__builtin_bit_cast(unsigned long long, c) & ~take_s);
+    return __builtin_bit_cast(double, bits ^ ((unsigned long long)(((qi + 1) >> 1) & 1) << 63));
+#else
     return (qi == 0) ? c : (qi == 1) ? -s : (qi == 2) ? -c : s;
+#endif
 }
 
 PSIM_QUAL double psim_pow4(double x) {

@@ -48,15 +48,22 @@ typedef struct {
     uint32_t v[4];
 } psim_u32x4;
 
+/* a ^ b ^ c: one instruction on gfx950 (truth table 0x96), which the compiler does not form itself */
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PSIM_XOR3(a, b, c) __builtin_amdgcn_bitop3_b32((a), (b), (c), 0x96)
+#else
+#define PSIM_XOR3(a, b, c) ((a) ^ (b) ^ (c))
+#endif
+
 /* One Philox4x32 round: two 32x32->64 products, then the S-box-free mixing
  * of the published algorithm. */
 PSIM_QUAL psim_u32x4 psim_philox_round(psim_u32x4 c, uint32_t k0, uint32_t k1) {
     const uint64_t p0 = (uint64_t)PSIM_PHILOX_M0 * (uint64_t)c.v[0];
     const uint64_t p1 = (uint64_t)PSIM_PHILOX_M1 * (uint64_t)c.v[2];
     psim_u32x4 r;
-    r.v[0] = (uint32_t)(p1 >> 32) ^ c.v[1] ^ k0;
+    r.v[0] = PSIM_XOR3((uint32_t)(p1 >> 32), c.v[1], k0);
     r.v[1] = (uint32_t)p1;
-    r.v[2] = (uint32_t)(p0 >> 32) ^ c.v[3] ^ k1;
+    r.v[2] = PSIM_XOR3((uint32_t)(p0 >> 32), c.v[3], k1);
     r.v[3] = (uint32_t)p0;
     return r;
 }
