@@ -9,8 +9,10 @@
 #include <chrono>
 #include <cmath>
 #include <ctime>
+#include <exception>
 #include <fstream>
 #include <iomanip>
+#include <mutex>
 #include <numeric>
 #include <sstream>
 #include <stdexcept>
@@ -776,6 +778,40 @@ std::pair<double, double> Model::setTemperatureBounds() {  // model.cpp:203-218
     return { *mn, *mx };
 }
 
+namespace {
+// fn(0) .. fn(n - 1) on up to `threads` host threads, the caller's among them; the first exception is
+// thrown again once all have ended.
+template <typename F>
+void parallelFor(std::size_t n, std::size_t threads, const F& fn) {
+    std::atomic<std::size_t> next{ 0 };
+    std::mutex mutex;
+    std::exception_ptr error;
+    auto work = [&]() {
+        try {
+            for (std::size_t i = next++; i < n; i = next++) { fn(i); }
+        } catch (...) {
+            next = n;
+            const std::lock_guard<std::mutex> lock(mutex);
+            if (!error) { error = std::current_exception(); }
+        }
+    };
+    std::vector<std::thread> pool;
+    try {
+        pool.reserve(threads);
+        for (std::size_t t = 1; t < std::min(n, threads); ++t) { pool.emplace_back(work); }
+    } catch (const std::exception&) {}  // no more threads or memory: those there are do the work
+    work();
+    for (auto& th : pool) { th.join(); }
+    if (error) { std::rethrow_exception(error); }
+}
+
+std::size_t hostThreads() { return std::max(1u, std::min(16u, std::thread::hardware_concurrency())); }
+
+// Tallies a host thread should have to interpret: one takes 0.1-0.3 us, a thread 20-40 us to start.
+// Interpreting the periodic L-shape (1e5 tallies) took 15 ms on one thread, 8 relaxations 25 ms.
+constexpr std::size_t TALLIES_PER_THREAD = 1024;
+}  // namespace
+
 std::vector<double> Model::findTemperature(const Sensor& s, double eff_energy, std::size_t start) const {
     const auto& energies = s.inc_energy;  // sensorInterpreter.cpp:80-112
     std::vector<double> temps(energies.size() - std::min(start, energies.size()));
@@ -847,11 +883,12 @@ void Model::runSimulation(psim_gpu_ctx* ctx, uint64_t seed) {  // model.cpp:141-
         simulator_.setEngine(ctx);
         const double eff0 = prepare(seed + run * RUN_SEED_STRIDE);
         simulator_.runSimulation(t_eq_, sensors_);
-        endRun(eff0, simulator_.totalPhonons(), simulator_.counters());
+        endRun(eff0, simulator_.totalPhonons(), simulator_.counters(), hostThreads());
     }
 }
 
-void Model::endRun(double eff0, int64_t total_phonons, const std::array<int64_t, PSIM_NUM_COUNTERS>& counters) {
+void Model::endRun(double eff0, int64_t total_phonons, const std::array<int64_t, PSIM_NUM_COUNTERS>& counters,
+    std::size_t threads) {
     RunRecord rec;
     rec.eff_energy = eff0;
     rec.total_phonons = total_phonons;
@@ -866,18 +903,21 @@ void Model::endRun(double eff0, int64_t total_phonons, const std::array<int64_t,
     }
     // Model::resetRequired (model.cpp:250-272): getFinalTemp with the budget's energy sets
     // each controller's t_steady_; refresh() then recomputes the energy per phonon with it.
+    threads = std::max<std::size_t>(1, std::min(threads, sensors_.size() * R / TALLIES_PER_THREAD));
     if (sim_type_ != SimulationType::Transient) {
-        for (auto& s : sensors_) {
+        parallelFor(sensors_.size(), threads, [&](std::size_t i) {
+            Sensor& s = sensors_[i];
             double ft = 0.;
             if (s.getArea() != 0.) {
                 const auto temps = findTemperature(s, eff0, start_step_);
                 ft = std::accumulate(temps.begin(), temps.end(), 0.) / static_cast<double>(R - start_step_);
             }
             s.setSteadyTemp(ft);
-        }
+        });
     }
     const double eff1 = getTotalInitialEnergy() / static_cast<double>(num_phonons_);
-    for (const auto& s : sensors_) { rec.measurements.push_back(scaleHeatParams(s, eff1)); }
+    rec.measurements.resize(sensors_.size());
+    parallelFor(sensors_.size(), threads, [&](std::size_t i) { rec.measurements[i] = scaleHeatParams(sensors_[i], eff1); });
     std::sort(rec.measurements.begin(), rec.measurements.end(),
         [](const auto& a, const auto& b) { return a.id < b.id; });
     runs_.push_back(std::move(rec));
@@ -923,8 +963,7 @@ void Model::runBatch(const std::vector<Model*>& models, psim_gpu_ctx* ctx, uint6
             } catch (const std::exception& e) { errors[i] = e.what(); }
         }
     };
-    const std::size_t n_threads = std::min<std::size_t>(models.size(),
-        std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+    const std::size_t n_threads = std::min(models.size(), hostThreads());
     std::vector<std::thread> pool;
     for (std::size_t t = 1; t < n_threads; ++t) { pool.emplace_back(work); }
     work();
@@ -1001,7 +1040,7 @@ void Model::runBatch(const std::vector<Model*>& models, psim_gpu_ctx* ctx, uint6
     }
     // Each model's slice of the tallies into its sensors, then the rest of its run.
     const std::array<int64_t, PSIM_NUM_COUNTERS> none{};
-    for (std::size_t i = 0; i < models.size(); ++i) {
+    parallelFor(models.size(), std::max<std::size_t>(1, std::min(n_threads, S * R / TALLIES_PER_THREAD)), [&](std::size_t i) {
         Model& m = *models[i];
         for (std::size_t si = 0; si < m.sensors_.size(); ++si) {
             const std::size_t row = static_cast<std::size_t>(sensor_base[i]) + si;
@@ -1010,9 +1049,9 @@ void Model::runBatch(const std::vector<Model*>& models, psim_gpu_ctx* ctx, uint6
                 m.sensors_[si].inc_flux[k] = { flux[2 * (row * R + k)], flux[2 * (row * R + k) + 1] };
             }
         }
-        m.endRun(eff0[i], m.simulator_.flat().params.total_phonons, none);
+        m.endRun(eff0[i], m.simulator_.flat().params.total_phonons, none, 1);
         m.simulator_.setStream(own_stream[i]);
-    }
+    });
 }
 
 void Model::exportResults(const std::filesystem::path& filepath, double time) const {  // outputManager.cpp:13-38

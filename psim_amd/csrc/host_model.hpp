@@ -298,8 +298,9 @@ private:
 
     Sensor& getSensor(std::size_t id);
     double prepare(uint64_t seed);
-    // The rest of one run once the sensors hold its tallies (model.cpp:161-181).
-    void endRun(double eff0, int64_t total_phonons, const std::array<int64_t, PSIM_NUM_COUNTERS>& counters);
+    // The rest of one run once the sensors hold its tallies (model.cpp:161-181), on up to `threads` host threads.
+    void endRun(double eff0, int64_t total_phonons, const std::array<int64_t, PSIM_NUM_COUNTERS>& counters,
+        std::size_t threads);
     double getTotalInitialEnergy() const;
     std::pair<double, double> setTemperatureBounds();
     std::vector<double> findTemperature(const Sensor& s, double eff_energy, std::size_t start) const;
