@@ -354,13 +354,13 @@ constexpr int TALLY_NONE = 0, TALLY_LDS = 1, TALLY_GLOBAL = 2;
 
 // Waves per SIMD the compiler must leave room for.  Without tally code the kernel fits 128 VGPRs
 // with a few values spilled to scratch, and four waves per SIMD hide more of its load latency;
-// with the tally code, 128 VGPRs spill in the tally path itself and three waves (~143 VGPRs) are
-// faster.
+// with the tally code, 128 VGPRs spill in the tally path itself and three waves (~142 VGPRs; asked for
+// two, the compiler takes 169 and gets them) are faster.
 #ifndef PSIM_UNTALLIED_WAVES_PER_EU
 #define PSIM_UNTALLIED_WAVES_PER_EU 4
 #endif
 #ifndef PSIM_TRANSPORT_WAVES_PER_EU
-#define PSIM_TRANSPORT_WAVES_PER_EU 2
+#define PSIM_TRANSPORT_WAVES_PER_EU 3
 #endif
 
 // Events of one wave, wave-uniform: counted from the stage masks in scalar registers.
@@ -382,9 +382,12 @@ enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_WALL = 
 // stage join the next in the same iteration.  Each lane still performs exactly the reference's
 // sequence of operations for its phonon, so trajectories are unchanged.
 // Bound: VALU issue (80% of the cycles in the untallied variant, 35 of 64 lanes active).  1e7
-// phonons of the L-shape: 1122 vector instructions per wave iteration, untallied launch 149.7 ms of
-// kernels in all, the run 158.7 ms; with reflections done inside the surface search, divisors not
-// shared, coefficients and buffer pointers spilled to vector lanes: 1580 and 200.2 ms.
+// phonons of the L-shape: 1122 vector instructions per wave iteration, the run 158.7 ms; with
+// reflections done inside the surface search, divisors not shared, coefficients and buffer pointers
+// spilled to vector lanes 1580 and 200.2 ms.  Runs that leave the chip part empty last as long as their
+// longest-lived phonons, whose events wait for loads half of the time: a stage's loads go out together
+// (pin) instead of each behind the branch that wants it.  Run of the L-shape 138.8 / 144.0 ms with /
+// without, bar of 5000 phonons 2.34 / 2.45, of 1000 sensors 35.6 / 37.7, 32 structures 121 / 125.
 // TALLY: the tally path of this launch (TALLY_NONE, TALLY_LDS, TALLY_GLOBAL).
 // MULTI: some source has a stream index or id base (a batch of models).  Otherwise a phonon's
 // id within its stream is its id and the stream word is the bare tag, so the single-model
@@ -773,6 +776,11 @@ transport_kernel(Args args) {
         if (state == S_SCAT || state == S_TTS || state == S_WALL) {
             const bool scat = state == S_SCAT, bounce = state == S_WALL && !passed;
             const Sensor& sensor = m.sensors[cur_sensor];
+            int mat = 0, table = 0;  // on their way while the first block is computed
+            if (scat) {
+                mat = sensor.material;
+                table = sensor.scatter_table;
+            }
             double nx = 0., ny = 0., spec = 1.;
             if (bounce) {
                 const Wall& w = m.walls[wall < 0 ? ~wall : wall];
@@ -793,9 +801,10 @@ transport_kernel(Args args) {
                 ++st.block;
             }
             bool turn;  // takes a new direction
+            pin(mat, table);
             if (scat) {
                 const bool resampled = u_a <= rates.a;
-                if (resampled) { resample(m, sensor.material, sensor.scatter_table, p, st); }
+                if (resampled) { resample(m, mat, table, p, st); }
                 turn = resampled ? u_a > rates.b : rates.impurity;
             } else {
                 turn = bounce && spec != 1. && !(u_a < spec);

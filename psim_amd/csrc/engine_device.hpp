@@ -144,6 +144,18 @@ __device__ __forceinline__ double recip(double d) { return psim_recip(d); }
 __device__ __forceinline__ double div_by(double n, double d, double r) { return psim_div_by(n, d, r); }
 __device__ __forceinline__ double div_normal(double n, double d) { return PSIM_DIV(n, d); }
 
+// Makes values arrive here: a load stays before the branches that follow, and goes out beside its
+// neighbours instead of where one branch or another first needs it.
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+    asm volatile("" : "+v"(x));
+}
+template <typename T, typename... U>
+__device__ __forceinline__ void pin(T& x, U&... more) {
+    pin(x);
+    pin(more...);
+}
+
 // ---- geometry (psim/src/geometry.cpp) ------------------------------------------------
 
 __device__ __forceinline__ double get_slope(double x1, double y1, double x2, double y2) {  // :325-327
@@ -251,15 +263,20 @@ enum : int { HIT_PASSED = 0, HIT_WALL = 1, HIT_ABSORBED = 2 };
 __device__ __forceinline__ int surface_hit(const Model& m, Ph& p, int& sensor, int& wall) {
     const Edge* e3 = m.edges + 3 * p.cell;
     const Edge &e0 = e3[0], &e1 = e3[1], &e2 = e3[2];
+    int2 sub0 = make_int2(e0.sub_begin, e0.n_sub), sub1 = make_int2(e1.sub_begin, e1.n_sub);
+    int2 sub2 = make_int2(e2.sub_begin, e2.n_sub);
     const bool on0 = on_line(e0.p1x, e0.p1y, e0.p2x, e0.p2y, p.px, p.py);
     const bool on1 = on_line(e1.p1x, e1.p1y, e1.p2x, e1.p2y, p.px, p.py);
     const bool on2 = on_line(e2.p1x, e2.p1y, e2.p2x, e2.p2y, p.px, p.py);
+    pin(sub0.x, sub0.y, sub1.x, sub1.y, sub2.x, sub2.y);
     if (!(on0 | on1 | on2)) { return HIT_PASSED; }
-    const int begin = on0 ? e0.sub_begin : on1 ? e1.sub_begin : e2.sub_begin;
-    const int n_sub = on0 ? e0.n_sub : on1 ? e1.n_sub : e2.n_sub;
     wall = 3 * p.cell + (on0 ? 0 : on1 ? 1 : 2);
+    const int begin = on0 ? sub0.x : on1 ? sub1.x : sub2.x;
+    const int n_sub = on0 ? sub0.y : on1 ? sub1.y : sub2.y;
     for (int i = begin; i < begin + n_sub; ++i) {
-        const Sub& s = m.subs[i];
+        Sub s = m.subs[i];  // whole, at once
+        pin(s.kind, s.target, s.target_sensor, s.same_material);
+        pin(s.start, s.duration, s.max_freq_la, s.max_freq_ta);
         if (!on_line(s.p1x, s.p1y, s.p2x, s.p2y, p.px, p.py)) { continue; }
         wall = m.sub_walls + i;
         if (s.kind == 0) {  // TransitionSurface::handlePhonon, surface.cpp:71-109
@@ -287,6 +304,8 @@ __device__ __forceinline__ int surface_hit(const Model& m, Ph& p, int& sensor, i
 // doesSegmentCrossLine :302-306 both ways, then the point) with the reference's operations and
 // roundings; what depends on the path alone (its box, slope, direction, the reciprocals of its
 // velocity) is computed once, and differences that only change sign are shared (negation is exact).
+// The predicates of all three edges come first, without branches, so that their loads share one wait;
+// the points of those crossed follow, with their slopes' loads in another.
 __device__ __forceinline__ bool find_impact(const Model& m, Ph& p, double time, double& out_time) {
     const double vx = p.dx * p.vel;
     const double vy = p.dy * p.vel;
@@ -304,32 +323,54 @@ __device__ __forceinline__ bool find_impact(const Model& m, Ph& p, double time, 
     const bool move_y = vy > VELOCITY_EPS || vy < -VELOCITY_EPS;
     const double rvx = recip(vx), rvy = recip(vy);  // used where move_x / move_y
     const Edge* e3 = m.edges + 3 * p.cell;
-    bool hit = false;
-    double ix = 0., iy = 0.;
+    double p1x[3], p1y[3], p2x[3], p2y[3];
     #pragma unroll
     for (int b = 0; b < 3; ++b) {
-        const Edge& s = e3[b];
-        const double p1x = s.p1x, p1y = s.p1y, p2x = s.p2x, p2y = s.p2y;
-        const bool box = ((p1x <= hix) | (p2x <= hix)) & ((p1x >= lox) | (p2x >= lox)) & ((p1y <= hiy) | (p2y <= hiy))
-                         & ((p1y >= loy) | (p2y >= loy));
-        const double ax = p2x - p1x, ay = p2y - p1y;
-        const double b1x = sx - p1x, b1y = sy - p1y, b2x = ex - p1x, b2y = ey - p1y;
+        p1x[b] = e3[b].p1x;
+        p1y[b] = e3[b].p1y;
+        p2x[b] = e3[b].p2x;
+        p2y[b] = e3[b].p2y;
+    }
+    bool reach[3];
+    #pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const bool box = ((p1x[b] <= hix) | (p2x[b] <= hix)) & ((p1x[b] >= lox) | (p2x[b] >= lox))
+                         & ((p1y[b] <= hiy) | (p2y[b] <= hiy)) & ((p1y[b] >= loy) | (p2y[b] >= loy));
+        const double ax = p2x[b] - p1x[b], ay = p2y[b] - p1y[b];
+        const double b1x = sx - p1x[b], b1y = sy - p1y[b], b2x = ex - p1x[b], b2y = ey - p1y[b];
         const double c1 = ax * b1y - b1x * ay, c2 = ax * b2y - b2x * ay;  // path ends against the edge's line
-        const double f2x = p2x - sx, f2y = p2y - sy;
+        const double f2x = p2x[b] - sx, f2y = p2y[b] - sy;
         const double d1 = ddx * b1y - b1x * ddy, d2 = f2x * ddy - ddx * f2y;  // edge ends against the path's
         const bool cross = ((fabs(c1) < GEOEPS) | (fabs(c2) < GEOEPS) | ((c1 < 0.) != (c2 < 0.)))
                            & ((fabs(d1) < GEOEPS) | (fabs(d2) < GEOEPS) | ((d1 < 0.) != (d2 < 0.)));
-        if (!(box & cross)) { continue; }
-        const double ss = s.slope, si = s.intercept;
-        const bool s_vert = s.vert != 0;
+        reach[b] = box & cross;
+    }
+    if (!(reach[0] | reach[1] | reach[2])) { return false; }
+    bool hit = false;
+    double ix = 0., iy = 0.;
+    double slope[3], icept[3];
+    int32_t vert[3];
+    #pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        slope[b] = e3[b].slope;
+        icept[b] = e3[b].intercept;
+        vert[b] = e3[b].vert;
+    }
+    pin(slope[0], slope[1], slope[2], icept[0], icept[1], icept[2]);
+    pin(vert[0], vert[1], vert[2]);
+    #pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        if (!reach[b]) { continue; }
+        const double ss = slope[b], si = icept[b];
+        const bool s_vert = vert[b] != 0;
         double qx, qy;
         if (o_vert && !s_vert) {  // the path vertical
-            const double mm = get_slope(p1x, p1y, p2x, p2y);
+            const double mm = get_slope(p1x[b], p1y[b], p2x[b], p2y[b]);
             qx = sx;
-            qy = mm * sx + (p1y - mm * p1x);
+            qy = mm * sx + (p1y[b] - mm * p1x[b]);
         } else {
             if (s_vert ? o_vert : rel_equals(ss, os)) { continue; }
-            qx = s_vert ? p1x : div_normal(oi - si, ss - os);
+            qx = s_vert ? p1x[b] : div_normal(oi - si, ss - os);
             qy = (s_vert ? os : ss) * qx + (s_vert ? oi : si);
         }
         const double gx = qx - sx, gy = qy - sy;
@@ -364,15 +405,17 @@ struct Rates {
 
 __device__ __forceinline__ double scatter_time(const Sensor& s, const Ph& p, double u, Rates& r) {
     const double freq = p.freq;
+    double b_l = s.b_l, t3 = s.t3, b_tn = s.b_tn, t4 = s.t4, b_tu = s.b_tu, b_i = s.b_i, w = s.w, tk = s.tk, r_tk = s.r_tk;
+    pin(b_l, t3, b_tn, t4, b_tu, b_i, w, tk, r_tk);
     double r0, r1;
     if (p.pol == POL_LA) {
-        r0 = s.b_l * freq * freq * s.t3;
+        r0 = b_l * freq * freq * t3;
         r1 = r0;
     } else {
-        r0 = (freq < s.w) ? s.b_tn * freq * s.t4 : 0.;
-        r1 = (freq >= s.w) ? s.b_tu * freq * freq / psim_sinh(div_by(HBAR * freq, s.tk, s.r_tk)) : 0.;
+        r0 = (freq < w) ? b_tn * freq * t4 : 0.;
+        r1 = (freq >= w) ? b_tu * freq * freq / psim_sinh(div_by(HBAR * freq, tk, r_tk)) : 0.;
     }
-    const double r2 = s.b_i * psim_pow4(freq);
+    const double r2 = b_i * psim_pow4(freq);
     const double total = 0. + r0 + r1 + r2;
     const double n = SCALING_FACTOR * -psim_log(u);
     r.impurity = r2 > 0.;
