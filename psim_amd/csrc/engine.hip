@@ -591,11 +591,12 @@ transport_kernel(Args args) {
     // is a phonon-step and, from adj on, a tally with the sensor and velocity of that moment.
     // Returns whether the step moved.
     auto advance_step = [&](double t, int32_t cap) -> bool {
-        int32_t k = p.step;
-        const int32_t est = (int32_t)(t * steps_per_time) - 1;  // a whole step below t: at or below the answer
-        if (est > k) { k = est < cap - 1 ? est : cap - 1; }
-        while (k + 1 < cap && boundary_time(k + 1) <= t) { ++k; }
-        if (k == p.step) { return false; }
+        // The estimate is within a step of the answer: N < 2^31 leaves its rounding error far below one.
+        int32_t k = (int32_t)(t * steps_per_time);
+        if (k >= cap) { k = cap - 1; }
+        const bool more = k + 1 < cap && boundary_time(k + 1) <= t, fewer = !(boundary_time(k) <= t);
+        k += (int32_t)more - (int32_t)fewer;
+        if (k <= p.step) { return false; }
         if constexpr (TALLY != TALLY_NONE) { tally_range(p.step + 1 > m.adj ? p.step + 1 : m.adj, k); }
         n_steps += (uint32_t)(k - p.step);
         p.step = k;
@@ -637,7 +638,7 @@ transport_kernel(Args args) {
                 state = S_PAUSED;
                 return;
             }
-            cap = cap_for(p.step);
+            cap = cap_len < m.N - cap ? cap + cap_len : m.N;  // cap_for(cap)
         } else {
             if (!m.phasor && tts == 0.) {
                 state = S_SCAT;

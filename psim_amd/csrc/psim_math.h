@@ -169,12 +169,8 @@ PSIM_QUAL double psim_sinh(double x) {
 /* cos(2 pi u); exact reduction of 4u into a quadrant and |f| <= 1/2. */
 PSIM_QUAL double psim_cos2pi(double u) {
     const double t = 4.0 * u; /* exact */
-    double q = floor(t);
-    double f = t - q; /* exact, in [0, 1) */
-    if (f > 0.5) {
-        f = f - 1.0;
-        q = q + 1.0;
-    }
+    const double q = ceil(t - 0.5); /* the difference is exact: t is a multiple of 2^-51 */
+    const double f = t - q; /* exact, in (-1/2, 1/2] */
     const double a = f * PSIM_K(PSIM_PIO2_HI) + f * PSIM_K(PSIM_PIO2_LO); /* |a| <= pi/4 */
     const double z = a * a;
     /* cos a = 1 - z/2 + z^2 (1/4! - z/6! + ... + z^6/16!) */
