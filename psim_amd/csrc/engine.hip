@@ -412,6 +412,11 @@ struct Args {
     uint32_t claim;  // work-queue items a wave claims per atomic
 };
 
+// Where the code lies matters where few waves hide the fetches of its 20 KB: with kernels at the
+// compiler's 256-byte boundaries the bar of 1e5 phonons took 10.8-13.8 ms from one build of this file to the
+// next, always 10.4-11.3 from 1 KB boundaries on (1, 4, 32 and 64 KB alike).
+constexpr int CODE_ALIGN = 4096;
+
 typedef const __attribute__((address_space(4))) Args* ArgsPtr;
 
 __device__ __forceinline__ ArgsPtr cold() {
@@ -421,7 +426,7 @@ __device__ __forceinline__ ArgsPtr cold() {
 }
 
 template <int TALLY, bool MULTI, int NT, typename FT>
-__global__ void __launch_bounds__(NT)
+__attribute__((aligned(CODE_ALIGN))) __global__ void __launch_bounds__(NT)
 __attribute__((amdgpu_waves_per_eu(TALLY == TALLY_NONE ? PSIM_UNTALLIED_WAVES_PER_EU : PSIM_TRANSPORT_WAVES_PER_EU)))
 transport_kernel(Args args) {
     const Model& m = args.m;
