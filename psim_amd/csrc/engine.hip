@@ -395,6 +395,9 @@ enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_WALL = 
 // both variants draw the same numbers for such a model.
 // NT: threads per block (128, 256 or 512), a launch shape the autotuner chooses.
 // FT: the flux tallies' element type, double or float (FP32 with Kahan-compensated sums).
+// TRI: every cell of the model is a triangle (Tri), as the host's all are; cells given edge by edge
+// otherwise have variants of their own, for 256-thread blocks (both in one kernel, chosen by a flag:
+// L-shape 128.9 ms, 127.1 without, bar of 1e5 phonons 11.8 and 10.9).
 // The kernel's one argument.  What the event loop reads all the time is taken from it once; the
 // rest (buffers that only refills, pauses and ends touch) is read again from the argument segment
 // where it is used (cold()): kept in scalar registers all along, those pointers crowded out the
@@ -425,7 +428,7 @@ __device__ __forceinline__ ArgsPtr cold() {
     return p;
 }
 
-template <int TALLY, bool MULTI, int NT, typename FT>
+template <int TALLY, bool MULTI, int NT, typename FT, bool TRI>
 __attribute__((aligned(CODE_ALIGN))) __global__ void __launch_bounds__(NT)
 __attribute__((amdgpu_waves_per_eu(TALLY == TALLY_NONE ? PSIM_UNTALLIED_WAVES_PER_EU : PSIM_TRANSPORT_WAVES_PER_EU)))
 transport_kernel(Args args) {
@@ -744,7 +747,7 @@ transport_kernel(Args args) {
     // One nextImpact of handleImpacts.
     auto stage_ni = [&]() {
         if (state == S_NI) {  // one nextImpact of handleImpacts
-            state = find_impact(m, p, drift_time - drifted, t_hit) ? S_COLL : S_END;
+            state = find_impact<TRI>(m, p, drift_time - drifted, t_hit) ? S_COLL : S_END;
         }
     };
     // The surface a hit lies on, and handleImpacts' bookkeeping.  A phonon that reflects goes on to
@@ -755,7 +758,7 @@ transport_kernel(Args args) {
             // the step of the moment of impact
             // the reference counts collisions per drift, and a drift ends at a boundary
             if (advance_step(age + (drifted + t_hit), cap)) { collisions = 0; }
-            const int hit = surface_hit(m, p, cur_sensor, wall);
+            const int hit = surface_hit<TRI>(m, p, cur_sensor, wall);
             if (hit == HIT_ABSORBED) {
                 state = S_DEAD + FATE_ABSORBED * 8;
             } else {
@@ -1209,6 +1212,7 @@ struct psim_gpu_ctx {
     std::string err;
     // model
     bool uploaded = false;
+    bool triangles = true;  // every cell's edges run from corner to corner (Tri)
     bool multi_stream = false;  // some source has a stream index or id base (a batch)
     psim_run_params params{};
     Model m{};
@@ -1388,7 +1392,7 @@ int32_t record_window_for(const psim_gpu_ctx* c) {
 // 77.4, with the narrow windows 88.1; periodic L-shape of 1.6e6 (180, was 60) 53.0 / 55.5 / 66.0 ms.
 constexpr int WIDE_BLOCK = 1024;
 int32_t wide_window_for(const psim_gpu_ctx* c) {
-    if (c->window > 0 || c->block != 256 || c->tally_fp32 || c->flight_cap <= 0
+    if (c->window > 0 || c->block != 256 || c->tally_fp32 || !c->triangles || c->flight_cap <= 0
         || c->params.total_phonons < (int64_t)c->n_cu * WIDE_BLOCK) {
         return 0;
     }
@@ -1478,7 +1482,7 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
         c->fate_cap = (int64_t)cap;
         c->gen++;
     }
-    const int tb = c->tally_fp32 ? 256 : c->block;  // transport threads per block (FP32 tallies: 256)
+    const int tb = c->tally_fp32 || !c->triangles ? 256 : c->block;  // transport threads per block
     const int64_t max_blocks = (int64_t)c->n_cu * c->blocks_per_cu, block_waves = tb / WAVE;
     const int64_t spread = std::min<int64_t>((int64_t)c->n_cu * SPREAD_WAVES_PER_CU, max_blocks * block_waves);
     const int lanes = (int)std::max<int64_t>(1, std::min<int64_t>(WAVE, (n + spread - 1) / spread));
@@ -1582,11 +1586,11 @@ int zero_fill(psim_gpu_ctx* c, std::initializer_list<std::pair<void*, size_t>> a
 }
 
 // One transport launch of the variant for this tally path, stream layout, block size and flux type.
-template <int NT, typename FT>
+template <int NT, typename FT, bool TRI>
 void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Args& args) {
     const dim3 g((unsigned)grid), b(NT);
 #define PSIM_TRANSPORT(T, M, F)                                                                              \
-    hipLaunchKernelGGL((transport_kernel<T, M, NT, F>), g, b, lds, c->stream, args)
+    hipLaunchKernelGGL((transport_kernel<T, M, NT, F, TRI>), g, b, lds, c->stream, args)
     // the untallied variant has no flux arrays: it is the same kernel for either flux type
     if (c->multi_stream) {
         if (tally == TALLY_NONE) {
@@ -1606,16 +1610,23 @@ void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const
 #undef PSIM_TRANSPORT
 }
 
-// The FP32 tally precision runs 256-thread blocks only (one more set of kernels, not three).
+// The FP32 tally precision and cells that are not triangles run 256-thread blocks only (one more set of
+// kernels each, not three).
 void launch_transport(psim_gpu_ctx* c, int tally, int grid, size_t lds, const Args& args) {
-    if (c->tally_fp32) {
-        launch_transport_nt<256, float>(c, tally, grid, lds, args);
+    if (!c->triangles) {
+        if (c->tally_fp32) {
+            launch_transport_nt<256, float, false>(c, tally, grid, lds, args);
+        } else {
+            launch_transport_nt<256, double, false>(c, tally, grid, lds, args);
+        }
+    } else if (c->tally_fp32) {
+        launch_transport_nt<256, float, true>(c, tally, grid, lds, args);
     } else if (c->block == 128) {
-        launch_transport_nt<128, double>(c, tally, grid, lds, args);
+        launch_transport_nt<128, double, true>(c, tally, grid, lds, args);
     } else if (c->block == 512) {
-        launch_transport_nt<512, double>(c, tally, grid, lds, args);
+        launch_transport_nt<512, double, true>(c, tally, grid, lds, args);
     } else {
-        launch_transport_nt<256, double>(c, tally, grid, lds, args);
+        launch_transport_nt<256, double, true>(c, tally, grid, lds, args);
     }
 }
 
@@ -1699,9 +1710,9 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
         if (rec && plan.wide) {
             const dim3 wg((unsigned)plan.rec_grid), wb(WIDE_BLOCK);
             if (c->multi_stream) {
-                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, true, WIDE_BLOCK, double>), wg, wb, lds, c->stream, args);
+                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, true, WIDE_BLOCK, double, true>), wg, wb, lds, c->stream, args);
             } else {
-                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, false, WIDE_BLOCK, double>), wg, wb, lds, c->stream, args);
+                hipLaunchKernelGGL((transport_kernel<TALLY_LDS, false, WIDE_BLOCK, double, true>), wg, wb, lds, c->stream, args);
             }
         } else {
             launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, args);
@@ -1999,9 +2010,24 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     std::vector<Wall> walls(edges.size() + (size_t)g->n_subs);
     for (size_t i = 0; i < edges.size(); ++i) {
         const psim_edge& e = g->edges[i];
-        edges[i] = Edge{ e.p1x, e.p1y, e.p2x, e.p2y, e.slope, e.intercept, rel_equals(e.p1x, e.p2x) ? 1 : 0, e.sub_begin,
+        const bool vert = rel_equals(e.p1x, e.p2x);
+        edges[i] = Edge{ e.p1x, e.p1y, e.p2x, e.p2y, vert ? e.p1x : e.slope, e.intercept, vert ? 1 : 0, e.sub_begin,
             e.n_trans + e.n_emit, 0 };
         walls[i] = Wall{ e.nx, e.ny, e.spec, 0. };
+    }
+    std::vector<Tri> tris((size_t)g->n_cells);
+    bool triangles = true;
+    for (size_t i = 0; i < tris.size(); ++i) {
+        tris[i] = Tri{};
+        for (int b = 0; b < 3; ++b) {
+            const Edge &e = edges[3 * i + (size_t)b], &next = edges[3 * i + (size_t)((b + 1) % 3)];
+            if (e.p2x != next.p1x || e.p2y != next.p1y || e.n_sub >= 1 << TRI_SUB_BITS) { triangles = false; }
+            tris[i].corner[b] = make_double2(e.p1x, e.p1y);
+            tris[i].sub_begin[b] = e.sub_begin;
+            tris[i].info |= ((uint32_t)e.n_sub & ((1u << TRI_SUB_BITS) - 1u)) << (TRI_SUB_BITS * b)
+                            | (uint32_t)e.vert << (3 * TRI_SUB_BITS + b);
+            tris[i].line[b] = make_double2(e.slope, e.intercept);
+        }
     }
     std::vector<Sub> subs((size_t)g->n_subs);
     for (size_t i = 0; i < subs.size(); ++i) {
@@ -2028,6 +2054,7 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     }
     PSIM_UPLOAD(cells, g->cells, g->n_cells);
     PSIM_UPLOAD(edges, edges.data(), edges.size());
+    PSIM_UPLOAD(tris, tris.data(), tris.size());
     PSIM_UPLOAD(walls, walls.data(), walls.size());
     PSIM_UPLOAD(subs, subs.data(), subs.size());
     PSIM_UPLOAD(sensors, sensors.data(), sensors.size());
@@ -2090,6 +2117,7 @@ int psim_gpu_upload(psim_gpu_ctx* c, const psim_geom* g, const psim_tables* t, c
     c->n_cells = g->n_cells;
     c->uploaded = true;
     c->multi_stream = multi;
+    c->triangles = triangles;
     c->gen++;
     return PSIM_OK;
 }

@@ -40,11 +40,24 @@ constexpr uint32_t META_NEG = 1u << 11;
 constexpr uint32_t META_IMPURITY = 1u << 12;
 constexpr int META_STREAM_SHIFT = 16;
 
-// One of a cell's three edges as the impact search and the surface stage read it: four 16-byte
-// loads.  `vert`: its ends have the same x up to rounding (rel_equals, tested once at upload).
+// A cell whose three edges run from corner to corner, as the impact search and the surface stage read
+// it: one cache line.  The corners stand once, so what the edges' tests need of each (its differences to
+// the path, the side of the path it lies on, its place against the path's box) is computed once, not for
+// the two edges that meet there.
+struct __attribute__((aligned(128))) Tri {
+    double2 corner[3];  // edge b runs from corner b to corner (b + 1) % 3
+    int32_t sub_begin[3];  // of each edge's sub-surfaces, transitions first
+    uint32_t info;  // their numbers, TRI_SUB_BITS bits each, then a bit for each vertical edge
+    double2 line[3];  // slope and intercept; a vertical edge's x instead of its slope
+    double pad_[2];
+};
+constexpr int TRI_SUB_BITS = 4;  // a model with an edge of more than 15 sub-surfaces uses Edge
+
+// One of a cell's three edges, for models whose cells are not all such triangles.
+// `vert`: its ends have the same x up to rounding (rel_equals, tested once at upload).
 struct __attribute__((aligned(16))) Edge {
     double p1x, p1y, p2x, p2y;
-    double slope, intercept;
+    double slope, intercept;  // a vertical edge's x instead of its slope
     int32_t vert;
     int32_t sub_begin, n_sub;  // its sub-surfaces, transitions first
     int32_t pad_;
@@ -89,6 +102,7 @@ struct __attribute__((aligned(16))) Table {
 
 struct Model {
     const psim_cell* __restrict__ cells;
+    const Tri* __restrict__ tris;  // [n_cells], read where every cell is one (TRI)
     const Edge* __restrict__ edges;  // [3 * n_cells]
     const Wall* __restrict__ walls;  // [3 * n_cells] of the edges, then [n_subs] of the sub-surfaces
     const Sub* __restrict__ subs;
@@ -260,19 +274,34 @@ __device__ __forceinline__ void redirect(double nx, double ny, Ph& p, psim_strea
 // the phonon into the cell it enters.
 enum : int { HIT_PASSED = 0, HIT_WALL = 1, HIT_ABSORBED = 2 };
 
+template <bool TRI>
 __device__ __forceinline__ int surface_hit(const Model& m, Ph& p, int& sensor, int& wall) {
-    const Edge* e3 = m.edges + 3 * p.cell;
-    const Edge &e0 = e3[0], &e1 = e3[1], &e2 = e3[2];
-    int2 sub0 = make_int2(e0.sub_begin, e0.n_sub), sub1 = make_int2(e1.sub_begin, e1.n_sub);
-    int2 sub2 = make_int2(e2.sub_begin, e2.n_sub);
-    const bool on0 = on_line(e0.p1x, e0.p1y, e0.p2x, e0.p2y, p.px, p.py);
-    const bool on1 = on_line(e1.p1x, e1.p1y, e1.p2x, e1.p2y, p.px, p.py);
-    const bool on2 = on_line(e2.p1x, e2.p1y, e2.p2x, e2.p2y, p.px, p.py);
-    pin(sub0.x, sub0.y, sub1.x, sub1.y, sub2.x, sub2.y);
-    if (!(on0 | on1 | on2)) { return HIT_PASSED; }
-    wall = 3 * p.cell + (on0 ? 0 : on1 ? 1 : 2);
-    const int begin = on0 ? sub0.x : on1 ? sub1.x : sub2.x;
-    const int n_sub = on0 ? sub0.y : on1 ? sub1.y : sub2.y;
+    int on = 3, begin = 0, n_sub = 0;
+    if constexpr (TRI) {
+        const Tri& t = m.tris[p.cell];
+        const double2 v0 = t.corner[0], v1 = t.corner[1], v2 = t.corner[2];
+        int32_t b0 = t.sub_begin[0], b1 = t.sub_begin[1], b2 = t.sub_begin[2];
+        uint32_t info = t.info;
+        const bool on0 = on_line(v0.x, v0.y, v1.x, v1.y, p.px, p.py);
+        const bool on1 = on_line(v1.x, v1.y, v2.x, v2.y, p.px, p.py);
+        const bool on2 = on_line(v2.x, v2.y, v0.x, v0.y, p.px, p.py);
+        pin(b0, b1, b2, info);
+        on = on0 ? 0 : on1 ? 1 : on2 ? 2 : 3;
+        begin = on0 ? b0 : on1 ? b1 : b2;
+        n_sub = (int)(info >> (TRI_SUB_BITS * on) & ((1u << TRI_SUB_BITS) - 1u));
+    } else {
+        #pragma unroll 1
+        for (int b = 2; b >= 0; --b) {
+            const Edge& e = m.edges[3 * p.cell + b];
+            if (on_line(e.p1x, e.p1y, e.p2x, e.p2y, p.px, p.py)) {
+                on = b;
+                begin = e.sub_begin;
+                n_sub = e.n_sub;
+            }
+        }
+    }
+    if (on == 3) { return HIT_PASSED; }
+    wall = 3 * p.cell + on;
     for (int i = begin; i < begin + n_sub; ++i) {
         Sub s = m.subs[i];  // whole, at once
         pin(s.kind, s.target, s.target_sensor, s.same_material);
@@ -306,6 +335,7 @@ __device__ __forceinline__ int surface_hit(const Model& m, Ph& p, int& sensor, i
 // velocity) is computed once, and differences that only change sign are shared (negation is exact).
 // The predicates of all three edges come first, without branches, so that their loads share one wait;
 // the points of those crossed follow, with their slopes' loads in another.
+template <bool TRI>
 __device__ __forceinline__ bool find_impact(const Model& m, Ph& p, double time, double& out_time) {
     const double vx = p.dx * p.vel;
     const double vy = p.dy * p.vel;
@@ -322,55 +352,98 @@ __device__ __forceinline__ bool find_impact(const Model& m, Ph& p, double time, 
     const bool move_x = vx > VELOCITY_EPS || vx < -VELOCITY_EPS;
     const bool move_y = vy > VELOCITY_EPS || vy < -VELOCITY_EPS;
     const double rvx = recip(vx), rvy = recip(vy);  // used where move_x / move_y
-    const Edge* e3 = m.edges + 3 * p.cell;
-    double p1x[3], p1y[3], p2x[3], p2y[3];
-    #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        p1x[b] = e3[b].p1x;
-        p1y[b] = e3[b].p1y;
-        p2x[b] = e3[b].p2x;
-        p2y[b] = e3[b].p2y;
-    }
     bool reach[3];
-    #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        const bool box = ((p1x[b] <= hix) | (p2x[b] <= hix)) & ((p1x[b] >= lox) | (p2x[b] >= lox))
-                         & ((p1y[b] <= hiy) | (p2y[b] <= hiy)) & ((p1y[b] >= loy) | (p2y[b] >= loy));
-        const double ax = p2x[b] - p1x[b], ay = p2y[b] - p1y[b];
-        const double b1x = sx - p1x[b], b1y = sy - p1y[b], b2x = ex - p1x[b], b2y = ey - p1y[b];
-        const double c1 = ax * b1y - b1x * ay, c2 = ax * b2y - b2x * ay;  // path ends against the edge's line
-        const double f2x = p2x[b] - sx, f2y = p2y[b] - sy;
-        const double d1 = ddx * b1y - b1x * ddy, d2 = f2x * ddy - ddx * f2y;  // edge ends against the path's
-        const bool cross = ((fabs(c1) < GEOEPS) | (fabs(c2) < GEOEPS) | ((c1 < 0.) != (c2 < 0.)))
-                           & ((fabs(d1) < GEOEPS) | (fabs(d2) < GEOEPS) | ((d1 < 0.) != (d2 < 0.)));
-        reach[b] = box & cross;
+    if constexpr (TRI) {
+        const Tri& t = m.tris[p.cell];
+        double vx[3], vy[3], bx[3], by[3];
+        bool near[3], side[3], left[3], right[3], below[3], above[3];
+        #pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double2 v = t.corner[k];
+            vx[k] = v.x;
+            vy[k] = v.y;
+        }
+        #pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            bx[k] = sx - vx[k];
+            by[k] = sy - vy[k];
+            const double d = ddx * by[k] - bx[k] * ddy;  // the corner against the path's line
+            near[k] = fabs(d) < GEOEPS;
+            side[k] = d < 0.;
+            left[k] = vx[k] <= hix;
+            right[k] = vx[k] >= lox;
+            below[k] = vy[k] <= hiy;
+            above[k] = vy[k] >= loy;
+        }
+        #pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const int e = (b + 1) % 3;
+            const bool box = (left[b] | left[e]) & (right[b] | right[e]) & (below[b] | below[e]) & (above[b] | above[e]);
+            const double ax = vx[e] - vx[b], ay = vy[e] - vy[b];
+            const double c1 = ax * by[b] - bx[b] * ay;  // path ends against the edge's line
+            const double c2 = ax * (ey - vy[b]) - (ex - vx[b]) * ay;
+            reach[b] = box & ((fabs(c1) < GEOEPS) | (fabs(c2) < GEOEPS) | ((c1 < 0.) != (c2 < 0.)))
+                       & (near[b] | near[e] | (side[b] != side[e]));
+        }
+    } else {
+        uint32_t set = 0;
+        #pragma unroll 1
+        for (int b = 0; b < 3; ++b) {
+            const Edge& s = m.edges[3 * p.cell + b];
+            const double p1x = s.p1x, p1y = s.p1y, p2x = s.p2x, p2y = s.p2y;
+            const bool box = ((p1x <= hix) | (p2x <= hix)) & ((p1x >= lox) | (p2x >= lox)) & ((p1y <= hiy) | (p2y <= hiy))
+                             & ((p1y >= loy) | (p2y >= loy));
+            const double ax = p2x - p1x, ay = p2y - p1y;
+            const double b1x = sx - p1x, b1y = sy - p1y, b2x = ex - p1x, b2y = ey - p1y;
+            const double c1 = ax * b1y - b1x * ay, c2 = ax * b2y - b2x * ay;
+            const double f2x = p2x - sx, f2y = p2y - sy;
+            const double d1 = ddx * b1y - b1x * ddy, d2 = f2x * ddy - ddx * f2y;
+            const bool cross = ((fabs(c1) < GEOEPS) | (fabs(c2) < GEOEPS) | ((c1 < 0.) != (c2 < 0.)))
+                               & ((fabs(d1) < GEOEPS) | (fabs(d2) < GEOEPS) | ((d1 < 0.) != (d2 < 0.)));
+            set |= (uint32_t)(box & cross) << b;
+        }
+        #pragma unroll
+        for (int b = 0; b < 3; ++b) { reach[b] = (set >> b & 1u) != 0; }
     }
     if (!(reach[0] | reach[1] | reach[2])) { return false; }
     bool hit = false;
     double ix = 0., iy = 0.;
     double slope[3], icept[3];
-    int32_t vert[3];
-    #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        slope[b] = e3[b].slope;
-        icept[b] = e3[b].intercept;
-        vert[b] = e3[b].vert;
+    uint32_t vert = 0;  // a bit for each edge
+    if constexpr (TRI) {
+        const Tri& t = m.tris[p.cell];
+        #pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const double2 l = t.line[b];
+            slope[b] = l.x;
+            icept[b] = l.y;
+        }
+        vert = t.info >> (3 * TRI_SUB_BITS);
+    } else {
+        #pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const Edge& s = m.edges[3 * p.cell + b];
+            slope[b] = s.slope;
+            icept[b] = s.intercept;
+            vert |= (uint32_t)s.vert << b;
+        }
     }
     pin(slope[0], slope[1], slope[2], icept[0], icept[1], icept[2]);
-    pin(vert[0], vert[1], vert[2]);
+    pin(vert);
     #pragma unroll
     for (int b = 0; b < 3; ++b) {
         if (!reach[b]) { continue; }
         const double ss = slope[b], si = icept[b];
-        const bool s_vert = vert[b] != 0;
+        const bool s_vert = (vert >> b & 1u) != 0;
         double qx, qy;
         if (o_vert && !s_vert) {  // the path vertical
-            const double mm = get_slope(p1x[b], p1y[b], p2x[b], p2y[b]);
+            const Edge& s = m.edges[3 * p.cell + b];
+            const double mm = get_slope(s.p1x, s.p1y, s.p2x, s.p2y);
             qx = sx;
-            qy = mm * sx + (p1y[b] - mm * p1x[b]);
+            qy = mm * sx + (s.p1y - mm * s.p1x);
         } else {
             if (s_vert ? o_vert : rel_equals(ss, os)) { continue; }
-            qx = s_vert ? p1x[b] : div_normal(oi - si, ss - os);
+            qx = s_vert ? ss : div_normal(oi - si, ss - os);
             qy = (s_vert ? os : ss) * qx + (s_vert ? oi : si);
         }
         const double gx = qx - sx, gy = qy - sy;
