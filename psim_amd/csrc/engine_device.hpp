@@ -476,10 +476,11 @@ struct Rates {
     bool impurity;
 };
 
-__device__ __forceinline__ double scatter_time(const Sensor& s, const Ph& p, double u, Rates& r) {
+template <bool UNI, typename S>  // S: Sensor, in global or (UNI) constant memory
+__device__ __forceinline__ double scatter_time(const S& s, const Ph& p, double u, Rates& r) {
     const double freq = p.freq;
     double b_l = s.b_l, t3 = s.t3, b_tn = s.b_tn, t4 = s.t4, b_tu = s.b_tu, b_i = s.b_i, w = s.w, tk = s.tk, r_tk = s.r_tk;
-    pin(b_l, t3, b_tn, t4, b_tu, b_i, w, tk, r_tk);
+    if constexpr (!UNI) { pin(b_l, t3, b_tn, t4, b_tu, b_i, w, tk, r_tk); }
     double r0, r1;
     if (p.pol == POL_LA) {
         r0 = b_l * freq * freq * t3;

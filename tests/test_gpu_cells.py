@@ -44,3 +44,28 @@ def test_cells_equal_the_oracle(teeth, sim_type, mode):
         # sums of the same terms in another order: at most ~1e4 terms a tally, each rounded to 2^-53 (2^-24)
         assert np.allclose(res.raw_flux, ref.flux, rtol=0, atol=rel * max(1.0, np.abs(ref.flux).max()))
     engine.close()
+
+
+# sensors alike (one record in scalar registers) and not (one of them starts at another temperature)
+@pytest.mark.parametrize("mode", ["hbm", "lds"])
+@pytest.mark.parametrize("alike", [True, False])
+def test_sensors_equal_the_oracle(alike, mode):
+    import oracle
+    import psim_amd
+    cfg = configs.linear_bar(num_sensors=5, num_phonons=20_000, num_measurements=100, sim_time=0.5, spec=0.5, sim_type=1,
+                             step_interval=10).to_dict()
+    if not alike:
+        cfg["sensors"][3]["t_init"] = 302.0
+    ref = oracle.Model(cfg).run(5, nthreads=8, fate=True)
+    engine = psim_amd.Engine(0)
+    engine.set_fate(True)
+    engine.set_tally_mode(mode)
+    model = psim_amd.Model(cfg)
+    model.run(engine, 5)
+    res = model.results(0)
+    for got, want in zip(engine.fetch_fate(model.budget()[1]), (ref.fate_step, ref.fate_cause, ref.fate_xy)):
+        assert np.array_equal(got, want)
+    assert res.counters == ref.counters and np.array_equal(res.counts, ref.counts)
+    # FP64 sums of the same terms in another order: at most ~1e4 terms a tally
+    assert np.allclose(res.raw_flux, ref.flux, rtol=0, atol=1e-11 * max(1.0, np.abs(ref.flux).max()))
+    engine.close()
