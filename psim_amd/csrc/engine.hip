@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(BIRTH_BLOCK) emit_kernel(Model m, Pool pool, i
             p.sign = src.sign;
             double birth = 0.;
             if (src.kind == 0) {  // CellOriginBuilder::operator()
-                resample(m, mat, src.table, p, st);
+                resample(m, m.tables[src.table], m.bins + mat * NBINS, p, st);
                 double r1, r2;
                 psim_urand2(&st, &r1, &r2);
                 if (r1 + r2 > 1.) {
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(BIRTH_BLOCK) emit_kernel(Model m, Pool pool, i
                 set_rand_direction(p, st);
             } else {  // SurfaceOriginBuilder::operator(), PhasorBuilder::operator()
                 birth = src.start + src.duration * psim_urand(&st);
-                resample(m, mat, src.table, p, st);
+                resample(m, m.tables[src.table], m.bins + mat * NBINS, p, st);
                 const double r1 = psim_urand(&st);
                 const double r2 = 1. - r1;
                 p.px = src.p1x * r1 + src.p2x * r2;
@@ -426,6 +426,19 @@ constexpr int CODE_ALIGN = 4096;
 typedef const __attribute__((address_space(4))) Args* ArgsPtr;
 typedef const __attribute__((address_space(4))) Sensor* SensorPtr;
 
+// LDS copies that a block of the UNI variants without LDS tallies takes of the one frequency table (20 KB)
+// and the material's bins (32 KB): a resample's four dependent lookups leave the L1, which answers 0.7
+// lookups per cycle, and wait a fraction of the time.  The bins only where the blocks that the registers
+// allow on a CU still fit beside each other: three of 256 threads with tallies in HBM, one of WIDE_BLOCK
+// without tallies, but not four of 256 (L-shape of 1e7 130.0 ms; with the table alone 119.4, without
+// either 124.9).  Bar of 1e5 phonons 10.4 ms, without 10.9.
+constexpr int WIDE_BLOCK = 1024;
+template <int TALLY, int NT, bool UNI>
+constexpr size_t staged_bytes() {
+    return !UNI || TALLY == TALLY_LDS ? 0
+           : NT == WIDE_BLOCK || (TALLY == TALLY_GLOBAL && NT >= 256) ? sizeof(Table) + sizeof(Bin) * NBINS : sizeof(Table);
+}
+
 __device__ __forceinline__ ArgsPtr cold() {
     ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));  // opaque: loads through it stay where they are written
@@ -440,7 +453,8 @@ transport_kernel(Args args) {
     const Tally& tally = args.tally;
     const int32_t k0 = args.k0, k1 = args.k1;
     const uint64_t seed = *args.seed_p;
-    extern __shared__ unsigned char lds_raw[];
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    constexpr bool STAGED = staged_bytes<TALLY, NT, UNI>() > 0, STAGED_BINS = staged_bytes<TALLY, NT, UNI>() > sizeof(Table);
     const int S = m.n_sensors;
     // LDS window tallies as difference arrays over the window's steps: a flight that passes
     // boundaries a..b adds its count and flux at row a and subtracts them at row b + 1, so its
@@ -454,6 +468,16 @@ transport_kernel(Args args) {
         lfx[i] = FT(0);
         lfy[i] = FT(0);
         lcnt[i] = 0;
+    }
+    if constexpr (STAGED) {
+        const uint4* from = reinterpret_cast<const uint4*>(m.tables + m.sensors[0].scatter_table);
+        uint4* to = reinterpret_cast<uint4*>(lds_raw);
+        for (int i = threadIdx.x; i < (int)(sizeof(Table) / 16); i += NT) { to[i] = from[i]; }
+        if constexpr (STAGED_BINS) {
+            from = reinterpret_cast<const uint4*>(m.bins + m.sensors[0].material * NBINS);
+            to += sizeof(Table) / 16;
+            for (int i = threadIdx.x; i < (int)(sizeof(Bin) * NBINS / 16); i += NT) { to[i] = from[i]; }
+        }
     }
     __syncthreads();
 
@@ -829,7 +853,16 @@ transport_kernel(Args args) {
             if constexpr (!UNI) { pin(mat, table); }
             if (scat) {
                 const bool resampled = u_a <= rates.a;
-                if (resampled) { resample(m, mat, table, p, st); }
+                if (resampled) {
+                    if constexpr (STAGED_BINS) {
+                        resample(m, *reinterpret_cast<const Table*>(lds_raw),
+                            reinterpret_cast<const Bin*>(lds_raw + sizeof(Table)), p, st);
+                    } else if constexpr (STAGED) {
+                        resample(m, *reinterpret_cast<const Table*>(lds_raw), m.bins + mat * NBINS, p, st);
+                    } else {
+                        resample(m, m.tables[table], m.bins + mat * NBINS, p, st);
+                    }
+                }
                 turn = resampled ? u_a > rates.b : rates.impurity;
             } else {
                 turn = bounce && spec != 1. && !(u_a < spec);
@@ -1411,7 +1444,6 @@ int32_t record_window_for(const psim_gpu_ctx* c) {
 // fill those blocks' lanes and whose models share a flight cap that fits twice; launch shapes set by
 // the caller are kept to.  Film of 3e6 phonons (240 steps a window, was 80) 70.7 ms, with 768 threads
 // 77.4, with the narrow windows 88.1; periodic L-shape of 1.6e6 (180, was 60) 53.0 / 55.5 / 66.0 ms.
-constexpr int WIDE_BLOCK = 1024;
 int32_t wide_window_for(const psim_gpu_ctx* c) {
     if (c->window > 0 || c->block != 256 || c->tally_fp32 || !c->triangles || c->flight_cap <= 0
         || c->params.total_phonons < (int64_t)c->n_cu * WIDE_BLOCK) {
@@ -1463,6 +1495,7 @@ struct RunPlan {
     int S = 0, grid = 1, lanes = WAVE;
     int rec_grid = 1;  // blocks of a recording launch with LDS tallies
     bool wide = false;
+    bool wide_free = false;  // untallied launches of one WIDE_BLOCK per CU
     int32_t W = 0;
     bool global_tally = false;
     std::vector<std::pair<int64_t, int64_t>> windows;
@@ -1583,6 +1616,10 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     plan.lanes = lanes;
     plan.rec_grid = rec_grid;
     plan.wide = wide != 0;
+    // runs that fill those blocks' lanes, in the default launch shape
+    plan.wide_free = c->one_sensor && c->triangles && !c->multi_stream && c->window == 0 && c->block == 256
+                     && c->blocks_per_cu == 8 && n >= (int64_t)c->n_cu * WIDE_BLOCK
+                     && (double)n * (double)N / ((double)c->n_cu * WIDE_BLOCK) < 2147483648.0;
     plan.steps_need = steps_need;
     plan.WS = WS;
     plan.W = W;
@@ -1614,9 +1651,11 @@ void launch_transport_nt(psim_gpu_ctx* c, int tally, int grid, size_t lds, const
         constexpr bool M = decltype(multi)::value, U = decltype(uni)::value;
         // the untallied variant has no flux arrays: it is the same kernel for either flux type
         if (tally == TALLY_NONE) {
-            hipLaunchKernelGGL((transport_kernel<TALLY_NONE, M, NT, double, TRI, U>), g, b, lds, c->stream, args);
+            hipLaunchKernelGGL((transport_kernel<TALLY_NONE, M, NT, double, TRI, U>), g, b, (staged_bytes<TALLY_NONE, NT, U>()),
+                c->stream, args);
         } else if (tally == TALLY_GLOBAL) {
-            hipLaunchKernelGGL((transport_kernel<TALLY_GLOBAL, M, NT, FT, TRI, U>), g, b, lds, c->stream, args);
+            hipLaunchKernelGGL((transport_kernel<TALLY_GLOBAL, M, NT, FT, TRI, U>), g, b, (staged_bytes<TALLY_GLOBAL, NT, U>()),
+                c->stream, args);
         } else {
             hipLaunchKernelGGL((transport_kernel<TALLY_LDS, M, NT, FT, TRI, U>), g, b, lds, c->stream, args);
         }
@@ -1736,6 +1775,9 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
             } else {
                 hipLaunchKernelGGL((transport_kernel<TALLY_LDS, false, WIDE_BLOCK, double, true, false>), wg, wb, lds, c->stream, args);
             }
+        } else if (!rec && plan.wide_free) {
+            hipLaunchKernelGGL((transport_kernel<TALLY_NONE, false, WIDE_BLOCK, double, true, true>), dim3((unsigned)c->n_cu),
+                dim3(WIDE_BLOCK), (staged_bytes<TALLY_NONE, WIDE_BLOCK, true>()), c->stream, args);
         } else {
             launch_transport(c, !rec ? TALLY_NONE : global_tally ? TALLY_GLOBAL : TALLY_LDS, grid, !rec ? 0 : lds, args);
         }

@@ -200,8 +200,9 @@ __host__ __device__ __forceinline__ bool rel_equals(double a, double b) {  // :1
 // g = 0..GUIDE) that index lies in [guide[g], guide[g + 1]] for g = floor(rand * GUIDE), which a
 // short scan finds: one dependent load in place of ten.  Tables that are not non-decreasing
 // have no guide and run the bisection.
-__device__ __forceinline__ void freq_index(const Table& t, bool guided, psim_stream& st, int& bin, int& pol) {
-    const double* __restrict__ cdf = t.cdf;
+template <typename T>
+__device__ __forceinline__ void freq_index(const T& t, bool guided, psim_stream& st, int& bin, int& pol) {
+    const auto* __restrict__ cdf = t.cdf;
     double rand, upol;  // the bisection's draw and the branch draw, one block
     psim_urand2(&st, &rand, &upol);
     int high;
@@ -238,10 +239,11 @@ __device__ __forceinline__ void freq_index(const Table& t, bool guided, psim_str
 
 // SensorController::initialUpdate / scatterUpdate with Material::getFreq, sensorController.cpp:28-55,
 // material.cpp:77-80
-__device__ __forceinline__ void resample(const Model& m, int mat, int table, Ph& p, psim_stream& st) {
+template <typename T, typename B>
+__device__ __forceinline__ void resample(const Model& m, const T& table, const B* bins, Ph& p, psim_stream& st) {
     int bin, pol;
-    freq_index(m.tables[table], m.guided != 0, st, bin, pol);
-    const Bin& bn = m.bins[mat * NBINS + bin];
+    freq_index(table, m.guided != 0, st, bin, pol);
+    const B& bn = bins[bin];
     const double f0 = bn.freq, vla = bn.vel_la, vta = bn.vel_ta, width = bn.width;
     p.freq = m.full ? f0 : f0 + (2. * psim_urand(&st) - 1.) * width / 2.;
     p.bin = bin;

@@ -69,3 +69,24 @@ def test_sensors_equal_the_oracle(alike, mode):
     # FP64 sums of the same terms in another order: at most ~1e4 terms a tally
     assert np.allclose(res.raw_flux, ref.flux, rtol=0, atol=1e-11 * max(1.0, np.abs(ref.flux).max()))
     engine.close()
+
+
+# one block of 1024 threads per CU from 1024 phonons per CU on (engine.hip, RunPlan::wide_free), tables in LDS
+@pytest.mark.parametrize("short", [1, 0])
+def test_wide_untallied_blocks_equal_the_oracle(short):
+    import oracle
+    import psim_amd
+    import torch
+    total = 1024 * torch.cuda.get_device_properties(0).multi_processor_count - short
+    cfg = configs.linear_bar(num_phonons=total - 1, num_measurements=60, sim_time=0.12, spec=0.5).to_dict()
+    ref = oracle.Model(cfg).run(5, nthreads=8, fate=True)
+    engine = psim_amd.Engine(0)
+    engine.set_fate(True)
+    model = psim_amd.Model(cfg)
+    model.run(engine, 5)
+    res = model.results(0)
+    assert abs(model.budget()[1] - total) <= 1
+    for got, want in zip(engine.fetch_fate(model.budget()[1]), (ref.fate_step, ref.fate_cause, ref.fate_xy)):
+        assert np.array_equal(got, want)
+    assert res.counters == ref.counters and np.array_equal(res.counts, ref.counts)
+    engine.close()
