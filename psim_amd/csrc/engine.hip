@@ -398,6 +398,9 @@ enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_WALL = 
 // UNI: all sensors have the same record, as in a model of one material that starts at one temperature: it
 // is read into scalar registers, where every lane used to load it for itself from L1, which answers
 // 0.7 lookups per cycle in this kernel.  L-shape 124.9 ms, 127.5 without, film of 3e6 phonons 54.4 and 55.5.
+// FULL: the first untallied launch of a full simulation (UNI, NT = WIDE_BLOCK): a frequency can only be a
+// bin's, so every block works out each bin's rates once, into its LDS (64 KB), in place of every scatter
+// for its own frequency.  L-shape of 1e7 phonons 111.6 ms, without 118.3.
 // TRI: every cell of the model is a triangle (Tri), as the host's all are; cells given edge by edge
 // otherwise have variants of their own, for 256-thread blocks (both in one kernel, chosen by a flag:
 // L-shape 128.9 ms, 127.1 without, bar of 1e5 phonons 11.8 and 10.9).
@@ -445,7 +448,7 @@ __device__ __forceinline__ ArgsPtr cold() {
     return p;
 }
 
-template <int TALLY, bool MULTI, int NT, typename FT, bool TRI, bool UNI>
+template <int TALLY, bool MULTI, int NT, typename FT, bool TRI, bool UNI, bool FULL = false>
 __attribute__((aligned(CODE_ALIGN))) __global__ void __launch_bounds__(NT)
 __attribute__((amdgpu_waves_per_eu(TALLY == TALLY_NONE ? PSIM_UNTALLIED_WAVES_PER_EU : PSIM_TRANSPORT_WAVES_PER_EU)))
 transport_kernel(Args args) {
@@ -477,6 +480,14 @@ transport_kernel(Args args) {
             from = reinterpret_cast<const uint4*>(m.bins + m.sensors[0].material * NBINS);
             to += sizeof(Table) / 16;
             for (int i = threadIdx.x; i < (int)(sizeof(Bin) * NBINS / 16); i += NT) { to[i] = from[i]; }
+        }
+    }
+    BinRates* bin_table = reinterpret_cast<BinRates*>(lds_raw + sizeof(Table) + sizeof(Bin) * NBINS);  // FULL
+    if constexpr (FULL) {
+        const Sensor& sensor = m.sensors[0];
+        for (int i = threadIdx.x; i < 2 * NBINS; i += NT) {
+            const int pol = i < NBINS ? 0 : 1;
+            bin_table[i] = bin_rates(sensor, m.bins[sensor.material * NBINS + i - pol * NBINS].freq, pol);
         }
     }
     __syncthreads();
@@ -754,6 +765,7 @@ transport_kernel(Args args) {
                     p.cell = L.cell;
                     cur_sensor = L.sensor;
                     p.step = (int32_t)(age / m.step_time);
+                    if constexpr (FULL) { p.bin = (int32_t)(meta & META_BIN); }
                 }
                 if (!MULTI) { sid = slot; }
                 if constexpr (UNI) {
@@ -904,7 +916,9 @@ transport_kernel(Args args) {
             } else if (scat && ++events > PSIM_MAX_EVENTS_PER_STEP) {  // begin_event's stall bound
                 state = S_DEAD + FATE_STALLED * 8;
             } else {  // tts is 0 here after a scatter, so begin_event would ask for a draw
-                if constexpr (UNI) {
+                if constexpr (FULL) {
+                    tts = scatter_time(bin_table[p.pol * NBINS + p.bin], scat ? u_b : u_a, rates);
+                } else if constexpr (UNI) {
                     tts = scatter_time<true>(*one_sensor(), p, scat ? u_b : u_a, rates);
                 } else {
                     tts = scatter_time<false>(m.sensors[cur_sensor], p, scat ? u_b : u_a, rates);
@@ -1775,6 +1789,9 @@ int enqueue_run(psim_gpu_ctx* c, const RunPlan& plan, bool eager) {
             } else {
                 hipLaunchKernelGGL((transport_kernel<TALLY_LDS, false, WIDE_BLOCK, double, true, false>), wg, wb, lds, c->stream, args);
             }
+        } else if (!rec && plan.wide_free && w == 0 && P.full && !P.phasor) {
+            hipLaunchKernelGGL((transport_kernel<TALLY_NONE, false, WIDE_BLOCK, double, true, true, true>), dim3((unsigned)c->n_cu),
+                dim3(WIDE_BLOCK), (staged_bytes<TALLY_NONE, WIDE_BLOCK, true>() + sizeof(BinRates) * 2 * NBINS), c->stream, args);
         } else if (!rec && plan.wide_free) {
             hipLaunchKernelGGL((transport_kernel<TALLY_NONE, false, WIDE_BLOCK, double, true, true>), dim3((unsigned)c->n_cu),
                 dim3(WIDE_BLOCK), (staged_bytes<TALLY_NONE, WIDE_BLOCK, true>()), c->stream, args);

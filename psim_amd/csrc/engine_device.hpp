@@ -35,6 +35,7 @@ enum : int { FATE_ABSORBED = 1, FATE_EXPIRED = 2, FATE_NOT_STARTED = 3, FATE_STA
 
 // Phonon record word: bits 0-9 frequency bin (emission pool), bit 10 TA, bit 11 negative sign, bit 12
 // impurities scatter it (Rates::impurity), bits 16-31 random-stream index (the model's index in a batch, 0 otherwise).
+constexpr uint32_t META_BIN = (1u << 10) - 1u;
 constexpr uint32_t META_TA = 1u << 10;
 constexpr uint32_t META_NEG = 1u << 11;
 constexpr uint32_t META_IMPURITY = 1u << 12;
@@ -479,20 +480,24 @@ struct Rates {
 };
 
 template <bool UNI, typename S>  // S: Sensor, in global or (UNI) constant memory
-__device__ __forceinline__ double scatter_time(const S& s, const Ph& p, double u, Rates& r) {
-    const double freq = p.freq;
+__device__ __forceinline__ double relax_rates(const S& s, double freq, int pol, double& r0, double& r1, double& r2) {
     double b_l = s.b_l, t3 = s.t3, b_tn = s.b_tn, t4 = s.t4, b_tu = s.b_tu, b_i = s.b_i, w = s.w, tk = s.tk, r_tk = s.r_tk;
     if constexpr (!UNI) { pin(b_l, t3, b_tn, t4, b_tu, b_i, w, tk, r_tk); }
-    double r0, r1;
-    if (p.pol == POL_LA) {
+    if (pol == POL_LA) {
         r0 = b_l * freq * freq * t3;
         r1 = r0;
     } else {
         r0 = (freq < w) ? b_tn * freq * t4 : 0.;
         r1 = (freq >= w) ? b_tu * freq * freq / psim_sinh(div_by(HBAR * freq, tk, r_tk)) : 0.;
     }
-    const double r2 = b_i * psim_pow4(freq);
-    const double total = 0. + r0 + r1 + r2;
+    r2 = b_i * psim_pow4(freq);
+    return 0. + r0 + r1 + r2;
+}
+
+template <bool UNI, typename S>
+__device__ __forceinline__ double scatter_time(const S& s, const Ph& p, double u, Rates& r) {
+    double r0, r1, r2;
+    const double total = relax_rates<UNI>(s, p.freq, p.pol, r0, r1, r2);
     const double n = SCALING_FACTOR * -psim_log(u);
     r.impurity = r2 > 0.;
     if (u > 0. && total > 1e-100 && total < 1e100) {
@@ -504,6 +509,32 @@ __device__ __forceinline__ double scatter_time(const S& s, const Ph& p, double u
     r.a = (r0 + r1) / total;
     r.b = r0 / total;
     return n / total;
+}
+
+// The same where a frequency can only be a bin's and all sensors are alike (full simulations of one
+// material): a block works out its bins' rates once, for both polarizations.
+struct __attribute__((aligned(16))) BinRates {
+    double a, b;  // b negative (-0 too) where impurities do not scatter
+    double total, r_total;  // the total's reciprocal, 0 near the ends of the exponent range
+};
+
+__device__ __forceinline__ BinRates bin_rates(const Sensor& s, double freq, int pol) {
+    double r0, r1, r2;
+    BinRates q;
+    q.total = relax_rates<false>(s, freq, pol, r0, r1, r2);
+    q.a = (r0 + r1) / q.total;
+    q.b = copysign(r0 / q.total, r2 > 0. ? 1. : -1.);
+    q.r_total = q.total > 1e-100 && q.total < 1e100 ? recip(q.total) : 0.;
+    return q;
+}
+
+__device__ __forceinline__ double scatter_time(const BinRates& q, double u, Rates& r) {
+    const double n = SCALING_FACTOR * -psim_log(u);
+    const double a = q.a, b = q.b, total = q.total, r_total = q.r_total;
+    r.a = a;
+    r.b = fabs(b);
+    r.impurity = !signbit(b);
+    return u > 0. && r_total != 0. ? div_by(n, total, r_total) : n / total;
 }
 
 // A new direction: Surface::redirectPhonon off a wall (surface.cpp:23-30), before its rotation to

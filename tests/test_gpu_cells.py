@@ -71,14 +71,18 @@ def test_sensors_equal_the_oracle(alike, mode):
     engine.close()
 
 
-# one block of 1024 threads per CU from 1024 phonons per CU on (engine.hip, RunPlan::wide_free), tables in LDS
-@pytest.mark.parametrize("short", [1, 0])
-def test_wide_untallied_blocks_equal_the_oracle(short):
+# one block of 1024 threads per CU from 1024 phonons per CU on (engine.hip, RunPlan::wide_free), tables in
+# LDS; in full simulations each bin's rates too, with impurities and without
+@pytest.mark.parametrize("short,t_eq,impurities", [(1, 300.0, True), (0, 300.0, True), (1, 0.0, True), (0, 0.0, True),
+                                                   (0, 0.0, False)])
+def test_wide_untallied_blocks_equal_the_oracle(short, t_eq, impurities):
     import oracle
     import psim_amd
-    import torch
-    total = 1024 * torch.cuda.get_device_properties(0).multi_processor_count - short
-    cfg = configs.linear_bar(num_phonons=total - 1, num_measurements=60, sim_time=0.12, spec=0.5).to_dict()
+    total = 1024 * 256 - 2 * short  # an MI355X has 256 CUs
+    cfg = configs.linear_bar(num_phonons=total, num_measurements=60, sim_time=0.12, spec=0.5, t_eq=t_eq).to_dict()
+    if not impurities:
+        for m in cfg["materials"]:
+            m["r_data"]["b_i"] = 0.0
     ref = oracle.Model(cfg).run(5, nthreads=8, fate=True)
     engine = psim_amd.Engine(0)
     engine.set_fate(True)
