@@ -1473,12 +1473,15 @@ int32_t free_window_for(const psim_gpu_ctx* c) { return c->window > 0 ? c->windo
 // Tally path of a run: LDS window partials for runs with enough phonons per sensor when enough
 // steps of tallies fit the LDS budget, else FP64 atomics into the HBM tallies (one launch for the
 // whole run).  psim_gpu_set_tally_mode forces either (LDS only where one step fits).
+// FP32 tallies keep to the rule by phonons per sensor alone: an HBM entry of theirs is a sum over the
+// whole run that nothing compensates (7.4e-6 of the largest tally, 7.0e-7 in LDS), and their segments
+// are not joined, so what LDS_MIN_PHONONS weighs is not theirs.
 bool use_global_tally(const psim_gpu_ctx* c) {
     const int64_t sensors = std::max(1, c->n_sensors);
     const int64_t lds_steps = LDS_TALLY_BYTES / (20 * sensors) - 1;
     if (c->tally_mode == PSIM_TALLY_HBM || lds_steps < 1) { return true; }
     if (c->tally_mode == PSIM_TALLY_LDS) { return false; }
-    if (c->params.total_phonons < LDS_MIN_PHONONS) { return true; }
+    if (!c->tally_fp32 && c->params.total_phonons < LDS_MIN_PHONONS) { return true; }
     if (wide_window_for(c) >= WIDE_LDS_STEPS) { return false; }
     return lds_steps < GLOBAL_TALLY_STEPS || c->params.total_phonons < LDS_MIN_PHONONS_PER_SENSOR * sensors;
 }
