@@ -325,10 +325,9 @@ def batch_bench(args) -> dict:
         _, _, gc = engine.run_graph(n_sensors, n_record, 30_001 + k)
         g_steps += gc["phonon_steps"]
         g_s += engine.last_timing()["run_ms"] / 1e3
-    # the same models one at a time (each its own upload and run), with the default launch shape
-    engine.set_window(0)
-    engine.set_grid(8)
-    engine.set_block(256)
+    # the same models one at a time (each its own upload and run), in the automatic launch shape
+    engine.close()
+    engine = psim_amd.Engine(0)
     seq_steps, seq_gpu = 0, 0.0
     for m in ([] if args.no_sequential else models):
         m.run(engine, 0)

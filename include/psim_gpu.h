@@ -230,15 +230,19 @@ int psim_gpu_last_timing(const psim_gpu_ctx* ctx, double* step_kernel_ms, int64_
  * flights pass its end, and their boundaries past it are tallied in HBM (same sums, slower). */
 int psim_gpu_set_window(psim_gpu_ctx* ctx, int32_t steps_per_launch);
 
-/* Engine tuning: transport blocks per compute unit (default 8). */
+/* Engine tuning: transport blocks per compute unit (default 8).  Until this or the block size is
+ * set, or the autotuner has chosen other values than the defaults, the shape is automatic: launches
+ * of a run of enough phonons may take one block of 1024 threads per compute unit instead.  Values
+ * set here, also the defaults, are kept to. */
 int psim_gpu_set_grid(psim_gpu_ctx* ctx, int32_t blocks_per_cu);
 
-/* Engine tuning: threads per transport block, 128, 256 (default) or 512.  No size changes a
- * result.  No counterpart in the reference. */
+/* Engine tuning: threads per transport block, 128, 256 (default) or 512; kept to once set, as the
+ * blocks per compute unit are.  No size changes a result.  No counterpart in the reference. */
 int psim_gpu_set_block(psim_gpu_ctx* ctx, int32_t threads);
 
 /* The launch shape in use: steps per untallied launch (0 = automatic), transport blocks per CU
- * and threads per transport block (any pointer may be NULL). */
+ * and threads per transport block (any pointer may be NULL).  The automatic shape reads as the
+ * defaults, 8 and 256. */
 int psim_gpu_get_launch_shape(const psim_gpu_ctx* ctx, int32_t* window, int32_t* blocks_per_cu, int32_t* block);
 
 /* Engine tuning: where recorded steps are tallied.  AUTO chooses by model size; LDS keeps
@@ -278,9 +282,9 @@ int psim_gpu_run_async(psim_gpu_ctx* ctx, uint64_t seed, void* stream);
 
 /* Autotuner: runs the uploaded model once for each candidate launch shape (untallied window
  * length 0 / 1024 / 256 and 8 or 3 transport blocks per CU at the current block size, then 128,
- * 256 and 512 threads per block at the best of those; none changes any result), keeps the fastest
- * in the context and reports it (the block size through psim_gpu_get_launch_shape).  No
- * counterpart in the reference. */
+ * 256 and 512 threads per block at the best of those; 8 blocks of 256 threads stand for the automatic
+ * shape; none changes any result), keeps the fastest in the context and reports it (the block size
+ * through psim_gpu_get_launch_shape).  No counterpart in the reference. */
 int psim_gpu_autotune(psim_gpu_ctx* ctx, uint64_t seed, int32_t* window, int32_t* blocks_per_cu, double* best_ms);
 
 /* ---- host model (C++17 behind the C ABI) ------------------------------------ */

@@ -1322,6 +1322,7 @@ struct psim_gpu_ctx {
     int32_t window = 0;
     int32_t blocks_per_cu = 8;  // transport grid: n_CU x blocks_per_cu blocks
     int32_t block = 256;  // threads per transport block
+    bool shape_set = false;  // the caller named the grid or the block, or the autotuner chose another than the defaults
     bool tally_fp32 = false;  // flux tallies in FP32 with Kahan-compensated sums (else FP64)
     int32_t tally_mode = PSIM_TALLY_AUTO;  // where recorded steps are tallied
     // seed of the current run, read by the kernels from device memory (pinned host staging copy)
@@ -1455,11 +1456,11 @@ int32_t record_window_for(const psim_gpu_ctx* c) {
 // which the last phonons finish, a sort and a reduction, so fewer windows run faster, and one block's
 // tallies per CU instead of up to eight are a quarter of the partials.  128 registers leave 16 waves
 // on the CU as four blocks of 256 would, which the smaller budget's tallies would not.  For runs that
-// fill those blocks' lanes and whose models share a flight cap that fits twice; launch shapes set by
-// the caller are kept to.  Film of 3e6 phonons (240 steps a window, was 80) 70.7 ms, with 768 threads
+// fill those blocks' lanes and whose models share a flight cap that fits twice; a grid or block set by
+// the caller (shape_set), also to the defaults, is kept to.  Film of 3e6 phonons (240 steps a window, was 80) 70.7 ms, with 768 threads
 // 77.4, with the narrow windows 88.1; periodic L-shape of 1.6e6 (180, was 60) 53.0 / 55.5 / 66.0 ms.
 int32_t wide_window_for(const psim_gpu_ctx* c) {
-    if (c->window > 0 || c->block != 256 || c->tally_fp32 || !c->triangles || c->flight_cap <= 0
+    if (c->window > 0 || c->shape_set || c->tally_fp32 || !c->triangles || c->flight_cap <= 0
         || c->params.total_phonons < (int64_t)c->n_cu * WIDE_BLOCK) {
         return 0;
     }
@@ -1633,9 +1634,9 @@ int prepare_run(psim_gpu_ctx* c, RunPlan& plan) {
     plan.lanes = lanes;
     plan.rec_grid = rec_grid;
     plan.wide = wide != 0;
-    // runs that fill those blocks' lanes, in the default launch shape
-    plan.wide_free = c->one_sensor && c->triangles && !c->multi_stream && c->window == 0 && c->block == 256
-                     && c->blocks_per_cu == 8 && n >= (int64_t)c->n_cu * WIDE_BLOCK
+    // runs that fill those blocks' lanes, in the automatic launch shape
+    plan.wide_free = c->one_sensor && c->triangles && !c->multi_stream && c->window == 0 && !c->shape_set
+                     && n >= (int64_t)c->n_cu * WIDE_BLOCK
                      && (double)n * (double)N / ((double)c->n_cu * WIDE_BLOCK) < 2147483648.0;
     plan.steps_need = steps_need;
     plan.WS = WS;
@@ -2273,15 +2274,17 @@ int psim_gpu_set_window(psim_gpu_ctx* c, int32_t steps) {
 
 int psim_gpu_set_grid(psim_gpu_ctx* c, int32_t blocks_per_cu) {
     if (!c || blocks_per_cu < 1 || blocks_per_cu > 64) { return PSIM_E_INVALID; }
-    if (c->blocks_per_cu != blocks_per_cu) { c->gen++; }
+    if (c->blocks_per_cu != blocks_per_cu || !c->shape_set) { c->gen++; }
     c->blocks_per_cu = blocks_per_cu;
+    c->shape_set = true;
     return PSIM_OK;
 }
 
 int psim_gpu_set_block(psim_gpu_ctx* c, int32_t threads) {
     if (!c || (threads != 128 && threads != 256 && threads != 512)) { return PSIM_E_INVALID; }
-    if (c->block != threads) { c->gen++; }
+    if (c->block != threads || !c->shape_set) { c->gen++; }
     c->block = threads;
+    c->shape_set = true;
     return PSIM_OK;
 }
 
@@ -2338,23 +2341,28 @@ int psim_gpu_autotune(psim_gpu_ctx* c, uint64_t seed, int32_t* window, int32_t* 
     // (0 = one launch; shorter ones re-sort the survivors by cell more often), the number of
     // transport blocks per CU and the threads per transport block.  Each candidate runs the
     // uploaded model once; the fastest is kept.  Window and grid are searched at the current block
-    // size, then the other block sizes at the best window and grid.
+    // size, then the other block sizes at the best window and grid.  The default grid and block stand
+    // for the automatic shape here, whatever was set before.
     const int32_t windows[] = { 0, 1024, 256 };
     const int32_t grids[] = { 8, 3 };
     const int32_t blocks[] = { 128, 256, 512 };
     const int32_t w0 = c->window, g0 = c->blocks_per_cu, b0 = c->block;
+    const bool set0 = c->shape_set;
+    const auto shape_set = [](int32_t g, int32_t b) { return g != 8 || b != 256; };
     double best = -1.;
     int32_t bw = w0, bg = g0, bb = b0;
     auto trial = [&](int32_t w, int32_t g, int32_t b) -> int {
         c->window = w;
         c->blocks_per_cu = g;
         c->block = b;
+        c->shape_set = shape_set(g, b);
         c->gen++;
         const int rc = run_impl(c, seed);
         if (rc != PSIM_OK) {
             c->window = w0;
             c->blocks_per_cu = g0;
             c->block = b0;
+            c->shape_set = set0;
             c->gen++;
             return rc;
         }
@@ -2379,6 +2387,7 @@ int psim_gpu_autotune(psim_gpu_ctx* c, uint64_t seed, int32_t* window, int32_t* 
     c->window = bw;
     c->blocks_per_cu = bg;
     c->block = bb;
+    c->shape_set = shape_set(bg, bb);
     c->gen++;
     if (window) { *window = bw; }
     if (blocks_per_cu) { *blocks_per_cu = bg; }
