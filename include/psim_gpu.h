@@ -259,8 +259,10 @@ int psim_gpu_set_tally_mode(psim_gpu_ctx* ctx, int32_t mode);
  * difference arrays and the HBM ones in FP32 (FP32 atomics), sums the window partials along the
  * steps and across blocks with Kahan compensation in FP32, and returns each tally as
  * sum - compensation in the same double arrays; integer counts are unaffected.  The trajectories
- * are those of FP64 (its launches are the narrow 256-thread ones), so a run of each on
- * one seed shows the error of the FP32 tallies against FP64.  No counterpart in the reference. */
+ * are those of FP64 (its recording launches are the narrow 256-thread ones; those before the first
+ * recorded step hold no flux and are FP64's), so a run of each on one seed shows the error of the
+ * FP32 tallies against FP64.  AUTO (psim_gpu_set_tally_mode) weighs phonons per sensor alone for it,
+ * because HBM entries are not compensated.  No counterpart in the reference. */
 #define PSIM_TALLY_FP64 0
 #define PSIM_TALLY_FP32_KAHAN 1
 int psim_gpu_set_tally_precision(psim_gpu_ctx* ctx, int32_t precision);

@@ -39,3 +39,16 @@ def test_small_fp32_runs_are_compensated(sensors, phonons, launches, bound):
     engine.close()
     assert n == launches
     _check(ref, res, bound)
+
+
+# steady state of enough phonons for 1024-thread blocks before the recorded steps (engine.hip,
+# RunPlan::wide_free), which hold no flux: full (each bin's rates in LDS) and deviational
+@pytest.mark.parametrize("t_eq", [0.0, 300.0])
+def test_fp32_run_after_wide_untallied_launch(t_eq):
+    import psim_amd
+    cfg = configs.lshape(num_phonons=300_000, num_measurements=1000, t_eq=t_eq).to_dict()
+    engine = psim_amd.Engine(0)
+    engine.set_tally_mode("lds")
+    ref, res, _ = _both(engine, psim_amd.Model(cfg), 6)
+    engine.close()
+    _check(ref, res, 2e-6)
