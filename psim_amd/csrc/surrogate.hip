@@ -2466,8 +2466,16 @@ int psim_mlp_forward(psim_mlp* h, const float* x, int32_t rows, float* y) {
     } else {
         if ((rc = load_batch(h, x, nullptr, rows)) != 0) { return rc; }
         if ((rc = forward(h, rows, false)) != 0) { return rc; }
-        hipLaunchKernelGGL(column0_kernel, dim3(ew_blocks(rows)), dim3(EW_BLOCK), 0, h->stream, h->zout, h->yout, rows, PAD_OUT);
+        // results that fit the pinned buffer, whose inputs' place is free here, without a copy operation
+        const size_t out_bytes = sizeof(float) * (size_t)rows;
+        float* out = out_bytes <= PINNED_BYTES ? h->h_x : h->yout;
+        hipLaunchKernelGGL(column0_kernel, dim3(ew_blocks(rows)), dim3(EW_BLOCK), 0, h->stream, h->zout, out, rows, PAD_OUT);
         MLP_CHECK(h, hipGetLastError());
+        if (out == h->h_x) {
+            MLP_CHECK(h, hipStreamSynchronize(h->stream));
+            std::memcpy(y, h->h_x, out_bytes);
+            return PSIM_OK;
+        }
     }
     MLP_CHECK(h, hipMemcpyAsync(y, h->yout, sizeof(float) * (size_t)rows, hipMemcpyDeviceToHost, h->stream));
     MLP_CHECK(h, hipStreamSynchronize(h->stream));
