@@ -44,20 +44,25 @@ constexpr int LDS_WIDE_BYTES = 160 * 1024;  // the same where one block has a CU
 constexpr int GLOBAL_TALLY_STEPS = 16;  // fewer LDS-tallied steps per window than this: HBM tallies
 // Fewer phonons than this in a run: HBM tallies too.  Every LDS window ends with a tail in which the last
 // phonons finish, a sort and a reduction; a run of HBM tallies has one.  Measured with wide windows
-// (wide_window_for), ms in LDS / in HBM, every step recorded: L-shape of 3e5 phonons 17.0 / 12.0, 6e5
-// 20.4 / 20.9, 1e6 25.7 / 30.8; film of 3e5 13.0 / 14.6, 6e5 15.1 / 22.9; bar of 6e5 19.8 / 16.5, 2e6
-// 27.5 / 36.6; bars of 1-4 sensors and 7e4-2.5e5 phonons 5.8-14.9 / 1.2-6.2.
+// (wide_window_for) and joined segments (MERGED), ms in LDS / in HBM, every step recorded: L-shape of 3e5
+// phonons 15.7 / 7.5, 6e5 16.6 / 9.9, 1e6 18.3 / 14.6; film of 3e5 13.7 / 14.5, 6e5 16.9 / 23.4, 1e6
+// 22.2 / 35.5; bar of 6e5 16.6 / 13.5, 1e6 19.2 / 17.2, 2e6 24.2 / 33.9; bar of 4 sensors and 7e4 or 2.5e5
+// phonons 21.2 / 4.4, 24.9 / 5.7.  The paths cross where the segments outweigh the windows, for a film
+// below 3e5 phonons, for L-shapes and bars above 1e6: one count for all is a compromise that costs films
+// of 3e5 to 6e5 up to 1.4 times their time in LDS, L-shapes and bars of 6e5 to 1e6 up to 1.7 times theirs
+// in HBM.
 constexpr int64_t LDS_MIN_PHONONS = 600000;
 // The same where the windows stay shorter than WIDE_LDS_STEPS steps, so that a run has many: the bar of
-// 100 sensors (69 steps a window) 40.9 / 27.9 at 1e4 phonons per sensor, 49.4 / 46.3 at 2e4.
+// 100 sensors (69 steps a window) 36.0 / 19.9 at 1e4 phonons per sensor, 43.0 / 35.0 at 2e4, 48.5 / 56.2
+// at 3e4.
 constexpr int32_t WIDE_LDS_STEPS = 128;
 constexpr int64_t LDS_MIN_PHONONS_PER_SENSOR = 30000;
 constexpr uint32_t QUEUE_CLAIM = 32;  // work-queue items a wave claims per atomic
 // A run of fewer phonons than the chip has lanes is as long as its longest-lived phonon: each event
 // waits for the one before.  An iteration costs a wave every stage that any of its lanes is in, so
 // such a run spreads over this many waves per CU (as many as fit with the untallied variant's
-// registers), each carrying fewer phonons, and a wave claims no phonon ahead of need.  Bar of 1e5
-// phonons: 64 / 32 / 16 / 8 / 1 lanes 13.2 / 12.1 / 11.6 / 12.2 / 16.5 ms (24 by this rule); of 5000:
+// registers), each carrying fewer phonons, and a wave claims no phonon ahead of need.  When the rule
+// came, bar of 1e5 phonons: 64 / 32 / 16 / 8 / 1 lanes 13.2 / 12.1 / 11.6 / 12.2 / 16.5 ms (24 by this rule); of 5000:
 // 4.0 / 3.6 / 3.4 / 2.7 / 2.6 ms (2 by this rule).  At 1e6 phonons fewer lanes lose (64 / 48 / 32:
 // 35.9 / 36.3 / 40.6 ms), and there claims of one item cost the atomics' latency (lshape 159 -> 231 ms).
 constexpr int SPREAD_WAVES_PER_CU = 16;
@@ -352,10 +357,10 @@ struct Lists {
 // FP64 atomics into the global tallies (too many sensors for LDS).
 constexpr int TALLY_NONE = 0, TALLY_LDS = 1, TALLY_GLOBAL = 2;
 
-// Waves per SIMD the compiler must leave room for.  Without tally code the kernel fits 128 VGPRs
-// with a few values spilled to scratch, and four waves per SIMD hide more of its load latency;
-// with the tally code, 128 VGPRs spill in the tally path itself and three waves (~142 VGPRs; asked for
-// two, the compiler takes 169 and gets them) are faster.
+// Waves per SIMD the compiler must leave room for.  Without tally code the kernel takes 124 VGPRs, and
+// four waves per SIMD hide more of its load latency; with LDS tallies it takes 127-130, with HBM tallies
+// 134-136, which four waves' 128 hold without spills to scratch and run no faster.  Blocks of WIDE_BLOCK
+// allow 128 whatever stands here.
 #ifndef PSIM_UNTALLIED_WAVES_PER_EU
 #define PSIM_UNTALLIED_WAVES_PER_EU 4
 #endif
@@ -381,19 +386,22 @@ enum : int { S_FETCH = 0, S_TTS = 1, S_NI = 2, S_COLL = 3, S_SCAT = 4, S_WALL = 
 // the wave runs them in that order, each for the lanes waiting in it, so lanes that finish one
 // stage join the next in the same iteration.  Each lane still performs exactly the reference's
 // sequence of operations for its phonon, so trajectories are unchanged.
-// Bound: VALU issue (80% of the cycles in the untallied variant, 35 of 64 lanes active).  1e7
-// phonons of the L-shape: 1122 vector instructions per wave iteration, the run 158.7 ms; with
-// reflections done inside the surface search, divisors not shared, coefficients and buffer pointers
-// spilled to vector lanes 1580 and 200.2 ms.  Runs that leave the chip part empty last as long as their
-// longest-lived phonons, whose events wait for loads half of the time: a stage's loads go out together
-// (pin) instead of each behind the branch that wants it.  Run of the L-shape 138.8 / 144.0 ms with /
-// without, bar of 5000 phonons 2.34 / 2.45, of 1000 sensors 35.6 / 37.7, 32 structures 121 / 125.
+// Bound: VALU issue.  1e7 phonons of the L-shape (a run of 111 ms): the untallied launch issues 5.0e10
+// vector instructions in 92 ms, one per 4.5 cycles of a SIMD, where FP64, 64-bit and multiply instructions
+// take 4.4-5; 33 of 64 lanes are active, 27 in the recording launches.  When reflections joined the draws,
+// divisors were shared and coefficients and buffer pointers stayed out of vector lanes, a wave iteration
+// went from 1580 vector instructions to 1122 and the run from 200.2 to 158.7 ms.  Runs that leave the chip
+// part empty last as long as their longest-lived phonons, whose events wait for loads half of the time: a
+// stage's loads go out together (pin) instead of each behind the branch that wants it (when that came,
+// L-shape 138.8 ms, without 144.0, bar of 5000 phonons 2.34 / 2.45, of 1000 sensors 35.6 / 37.7, 32
+// structures 121 / 125).
 // TALLY: the tally path of this launch (TALLY_NONE, TALLY_LDS, TALLY_GLOBAL).
 // MULTI: some source has a stream index or id base (a batch of models).  Otherwise a phonon's
 // id within its stream is its id and the stream word is the bare tag, so the single-model
 // variant neither loads nor stores the per-phonon stream id and keeps that word a constant;
 // both variants draw the same numbers for such a model.
-// NT: threads per block (128, 256 or 512), a launch shape the autotuner chooses.
+// NT: threads per block: 256, or 128 or 512 where the caller or the autotuner asks for them; WIDE_BLOCK
+// where one block takes a CU (wide_window_for, RunPlan::wide_free).
 // FT: the flux tallies' element type, double or float (FP32 with Kahan-compensated sums).
 // UNI: all sensors have the same record, as in a model of one material that starts at one temperature: it
 // is read into scalar registers, where every lane used to load it for itself from L1, which answers
@@ -1457,8 +1465,9 @@ int32_t record_window_for(const psim_gpu_ctx* c) {
 // tallies per CU instead of up to eight are a quarter of the partials.  128 registers leave 16 waves
 // on the CU as four blocks of 256 would, which the smaller budget's tallies would not.  For runs that
 // fill those blocks' lanes and whose models share a flight cap that fits twice; a grid or block set by
-// the caller (shape_set), also to the defaults, is kept to.  Film of 3e6 phonons (240 steps a window, was 80) 70.7 ms, with 768 threads
-// 77.4, with the narrow windows 88.1; periodic L-shape of 1.6e6 (180, was 60) 53.0 / 55.5 / 66.0 ms.
+// the caller (shape_set), also to the defaults, is kept to.  Film of 3e6 phonons (240 steps a window, for
+// 80) 52.7 ms, with the narrow windows 68.1; periodic L-shape of 1.6e6 (180, for 60) 21.2 and 29.0.
+// Blocks of 768 threads were a tenth slower than of 1024.
 int32_t wide_window_for(const psim_gpu_ctx* c) {
     if (c->window > 0 || c->shape_set || c->tally_fp32 || !c->triangles || c->flight_cap <= 0
         || c->params.total_phonons < (int64_t)c->n_cu * WIDE_BLOCK) {

@@ -2449,7 +2449,8 @@ int psim_mlp_forward(psim_mlp* h, const float* x, int32_t rows, float* y) {
         }
         if ((rc = ensure_io(h, rows)) != 0) { return rc; }
         // large inputs in equal pieces, each computed while the next is copied (100003 rows in four
-        // pieces 491 us, as one 556 us, of which 154 are the kernel's)
+        // pieces 491 us, as one 556 us, of which 154 are the kernel's; with a new input and result
+        // array for every call 620 us)
         const int pieces = (rows + COPY_ROWS - 1) / COPY_ROWS;
         const int piece = ((rows + pieces - 1) / pieces + BATCH_ROUND - 1) / BATCH_ROUND * BATCH_ROUND;
         const hipStream_t cs = pieces > 1 ? h->copies : h->stream;
@@ -2467,6 +2468,7 @@ int psim_mlp_forward(psim_mlp* h, const float* x, int32_t rows, float* y) {
         if ((rc = load_batch(h, x, nullptr, rows)) != 0) { return rc; }
         if ((rc = forward(h, rows, false)) != 0) { return rc; }
         // results that fit the pinned buffer, whose inputs' place is free here, without a copy operation
+        // (1024 x 3, 1 row 50 us, copied 71; 600 -> 512 x 3, 3000 rows 267 us, copied 291)
         const size_t out_bytes = sizeof(float) * (size_t)rows;
         float* out = out_bytes <= PINNED_BYTES ? h->h_x : h->yout;
         hipLaunchKernelGGL(column0_kernel, dim3(ew_blocks(rows)), dim3(EW_BLOCK), 0, h->stream, h->zout, out, rows, PAD_OUT);
