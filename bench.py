@@ -9,11 +9,12 @@ specularity 0.3, T_init 300 K), full (non-deviational) mode, 1e7 phonons, FP64 t
   value      phonon-steps per second of the timed runs (a phonon-step is one live phonon carried
              across one measurement interval: the reference's ++step at
              psim/src/modelSimulator.cpp:182-183), with the model already resident in HBM.
-  roofline   the transport kernel against the step-synchronous HBM model of this path: 120 bytes
-             per phonon-step (the phonon record read and written once per step) over its
-             HIP-event time on the engine stream.  What the counters show limits it (`limiter`,
-             VALU issue, and the measured HBM bytes per phonon-step) is copied from profiles/,
-             labelled with the engine commit it was measured on and whether that is this tree's.
+  roofline   the transport kernel against what limits it, the issue of vector instructions: the
+             instructions per phonon-step that the counters show on this workload (copied from
+             profiles/, labelled with the engine commit they were measured on and whether that is
+             this tree's) over its HIP-event time on the engine stream, against one per SIMD and
+             four cycles.  `step_synchronous` is no bound: the rate at which a design that reads and
+             writes every phonon's record once a step would have to move memory to keep up.
   cpu_baseline  the reference psim (oracle/_ref/psim_ref, built from the reference sources) on
              a bounded sample of the same workload (1e5 phonons): one process per CPU of the
              job's share (the affinity set, at most 16) started together, their aggregate rate
@@ -71,6 +72,8 @@ sys.path.insert(0, ROOT)
 
 BYTES_PER_PHONON_STEP = 120.0
 HBM_PEAK_GBPS = 8000.0
+# 256 CUs x 4 SIMDs at 2.4 GHz, an FP64 instruction of a wave taking four cycles (1e9 per second)
+VALU_ISSUE_PEAK = 256 * 4 * 2.4 / 4.0
 ENGINE_SOURCES = ("psim_amd/csrc/engine.hip", "psim_amd/csrc/engine_device.hpp", "psim_amd/csrc/psim_rng.h",
                   "psim_amd/csrc/psim_math.h", "include/psim_gpu.h")
 
@@ -590,7 +593,7 @@ def main() -> int:
         launches += tm["step_launches"]
     wall = time.perf_counter() - t0
     value = steps_total / wall
-    achieved = BYTES_PER_PHONON_STEP * steps_total / (kernel_ms / 1e3) / 1e9
+    nominal = BYTES_PER_PHONON_STEP * steps_total / (kernel_ms / 1e3) / 1e9
     line = {
         "metric": "phonon-steps/s",
         "value": value,
@@ -608,18 +611,19 @@ def main() -> int:
         "method": "phonons fly across the measurement boundaries; each boundary passed is counted as a phonon-step "
                   "and, when recorded, tallied with the phonon's sensor and velocity of that moment",
         "roofline": {
-            # the step-synchronous HBM model of this path; what the counters show limits the
-            # kernel (VALU issue) is `limiter` below
-            "bound": "hbm",
-            "model": "120 algorithmic bytes per phonon-step: one 60-byte SoA phonon record read and written "
-                     "per measurement step",
+            # achieved and frac need this workload's instruction counts (below)
+            "bound": "valu-issue",
+            "model": "vector instructions of the transport launches against one per SIMD and four cycles",
             "kernel": "transport_kernel",
-            "achieved": achieved,
-            "peak": HBM_PEAK_GBPS,
-            "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBPS,
+            "achieved": None,
+            "peak": VALU_ISSUE_PEAK,
+            "unit": "1e9 wave instructions/s",
+            "frac": None,
             "traffic": None,
-            "bytes_per_phonon_step": BYTES_PER_PHONON_STEP,
+            "step_synchronous": {"bytes_per_phonon_step": BYTES_PER_PHONON_STEP, "nominal_gbps": nominal,
+                                 "over_hbm_peak": nominal / HBM_PEAK_GBPS,
+                                 "note": "what a design that reads and writes a 60-byte record per phonon and step "
+                                         "would have to move; this engine keeps the record in registers"},
             "kernel_ms_per_launch": kernel_ms / max(1, launches),
             "launches": launches,
         },
@@ -639,6 +643,9 @@ def main() -> int:
             per_launch = steps_total / max(1, launches)
             line["roofline"]["traffic"] = copied["traffic"]["bytes_per_phonon_step"] * per_launch
             line["roofline"]["traffic_bytes_per_phonon_step"] = copied["traffic"]["bytes_per_phonon_step"]
+            achieved = copied["issue"]["valu_insts_per_phonon_step"] * steps_total / (kernel_ms / 1e3) / 1e9
+            line["roofline"]["achieved"] = achieved
+            line["roofline"]["frac"] = achieved / VALU_ISSUE_PEAK
             line["roofline"]["limiter"] = copied["limiter"]
             line["roofline"]["issue"] = copied["issue"]
             line["roofline"]["counters_copied_from"] = {
